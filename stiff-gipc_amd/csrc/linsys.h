@@ -182,7 +182,7 @@ class Mas
                      const double* rz_prev, const double* pAp, float* z, double* rz_out,
                      double* zero0, double* zero1, const int* done, hipStream_t s,
                      bool defer_rz = false);
-    // workgroups of the collect launch (partials of its rz set)
+    // workgroups of the apply's last launch (partials of its rz set)
     int collect_blocks() const { return (int)grid_for(nv_, 256); }
 
     int levels() const { return L_; }
@@ -203,6 +203,11 @@ class Mas
     void apply_fused_t(V* x, V* r, const V* p, const V* Ap, const double* rz_prev,
                        const double* pap, V* z, double* rz_out, double* zero0, double* zero1,
                        const int* done, hipStream_t s, bool defer_rz);
+    template <typename T, typename V>
+    void apply_levels(const T* inv, T* R, T* Z, V* x, V* r, const V* p, const V* Ap,
+                      const double* rz_prev, const double* pap, V* z, double* rz_out,
+                      double* zero0, double* zero1, const int* done, hipStream_t s,
+                      bool defer_rz);
     void cluster_level(int level, hipStream_t s);
     void assemble(const SysView& S, hipStream_t s);
     void invert(hipStream_t s);
@@ -230,6 +235,7 @@ class Mas
     DBuf<int>      bank_first_; // global bank -> first next-level global id
     DBuf<int>      bank_ncl_;   // global bank -> number of next-level nodes
     DBuf<int>      child_bank_; // global id (levels >= 1) -> bank holding its members
+    DBuf<unsigned> child_mask_; // ... and the members' lanes in that bank
     size_t         nbanks_alloc_ = 0;
     MasGalerkin    galerkin_;
 };

@@ -220,7 +220,8 @@ __global__ void __launch_bounds__(256) k_assign(int level, int total_map, const 
                                                 const int* __restrict__ bank_cnt,
                                                 int* __restrict__ newid, int* __restrict__ going_next,
                                                 int* __restrict__ bank_first, int* __restrict__ bank_ncl,
-                                                int* __restrict__ child_bank)
+                                                int* __restrict__ child_bank,
+                                                unsigned* __restrict__ child_mask)
 {
     int  t      = blockIdx.x * blockDim.x + threadIdx.x;
     int  lane16 = t & 15;
@@ -251,9 +252,10 @@ __global__ void __launch_bounds__(256) k_assign(int level, int total_map, const 
     int id   = bank_prefix[bank] + __popc(grp & ((1u << e) - 1u));
     newid[t] = id;
     going_next[off_l + t] = off_n + id;
-    // the bank holding the members of the new node (every member stores the
-    // same value)
+    // the bank holding the members of the new node and their lanes in it
+    // (every member stores the same values)
     child_bank[off_n + id] = (off_l >> 4) + bank;
+    child_mask[off_n + id] = c;
 }
 
 // per fine vertex: node id at level l+1 and its chain entry
@@ -655,212 +657,264 @@ __global__ void __launch_bounds__(64) k_mas_lx(int bank0, int node0, int count,
         restrict_bank(Rc, rv, valid ? going_next[g] : -1, bank_first[gb], bank_ncl[gb], R);
 }
 
-// The coarse levels from lt up (the tail), in one launch: every workgroup
-// loads R_lt (stored complete by the level lt-1 launch), sums the higher
-// levels' R in LDS and gives one wave to each of its share of the tail banks
-// (each wave at most one bank: the launch has ceil(banks / kCoarseWaves)
-// workgroups, each restricting R redundantly).  Everything it reads from
-// global memory -- this wave's bank inverse (FP32), R_lt, goingNext and the
-// member banks over the tail's node span -- is requested in one batch per
-// thread before the first use, so the chain is one memory round trip, the
-// LDS restriction and the product.  Every cluster sum adds the cluster's
-// member nodes in node order: the members of cluster p of level l+1 are the
-// nodes of the level-l bank cb[p] whose parent is p.
-constexpr int kCoarseWaves = 16;
-constexpr int kTailBanks   = 128;   // a level with at most this many banks may start the tail
-constexpr int kTailNodes   = 4096;  // node span of the tail levels (a multiple of 16)
-constexpr int kTailThreads = 64 * kCoarseWaves;
-constexpr int kTailSpanPer = kTailNodes / kTailThreads;      // span entries per thread
-constexpr int kTailRPer    = 3 * kTailNodes / kTailThreads;  // R values per thread
-struct LevelTable
+// The end of the apply, one launch: the coarse levels from lt up (the tail)
+// and z = sum over levels.  A workgroup owns kFinThreads consecutive vertices,
+// which descend from few tail nodes (16 vertices share a level-1 node, 256 a
+// level-2 node), so it needs few rows of the tail inverses: it loads R_lt whole
+// (stored complete by the launch before), sums the higher levels' R in LDS,
+// multiplies the rows of its own distinct tail nodes, and adds each vertex's
+// levels in order.  The tail's R is restricted redundantly by every
+// workgroup, which costs less than a launch of its own between the levels and
+// the sum: dependent memory round trips (about a microsecond each after a
+// launch), not bytes, bound both.  Every cluster sum adds the cluster's
+// members in node order.  Against a tail launch of its own followed by the
+// sum (a round of products per level for every tail bank, then a gather): per
+// PCG iteration 33.2 to 25.7 us on 6,480 rows (FP64 MAS), 41.3 to 38.4 us on
+// 46,656 rows, 106.8 to 102.3 us on 173,225 rows.
+constexpr int kFinThreads = 256;
+constexpr int kMaxLevels  = 6;          // compute_num_levels' bound
+constexpr int kFinLds     = 64 * 1024;  // LDS of one workgroup at most (two per CU)
+struct TailPlan
 {
-    int count[24];
-    int off[24];
+    int lt    = 0;  // first tail level (L: no tail)
+    int base  = 0;  // global id of the tail's first node (a multiple of 16)
+    int span  = 0;  // padded nodes of the tail
+    int first = 0;  // padded nodes of level lt
+    int count[kMaxLevels] = {};
+    int off[kMaxLevels]   = {};
 };
 
+// LDS of k_mas_finish: R of the tail, the products of the distinct tail nodes
+// (three components per node, at most kFinThreads nodes per level), their
+// list, the members of the nodes above lt
 template <typename T>
-__global__ void __launch_bounds__(kTailThreads)
-    k_mas_coarse(LevelTable lv, int L, int lt, const T* __restrict__ inv,
-                 const int* __restrict__ going_next, const int* __restrict__ child_bank,
-                 const T* __restrict__ R, T* __restrict__ Z, const int* __restrict__ done)
+static size_t finish_lds(int span, int levels)
 {
-    if(done && *done)
-        return;
-    __shared__ T             Rs[3 * kTailNodes];
-    __shared__ int           up[kTailNodes];
-    __shared__ unsigned char cb[kTailNodes];  // member bank of a node above lt, minus b0
-    const int w    = threadIdx.x >> 6;
-    const int t    = threadIdx.x & 63;
-    const int base = lv.off[lt];
-    const int span = lv.off[L - 1] + lv.count[L - 1] - base;
-    const int nb   = (span + BANK - 1) / BANK;  // banks of the tail levels
-    const int b0   = base / BANK;
-    const int bi   = blockIdx.x * kCoarseWaves + w;
-    const int nr   = 3 * lv.count[lt];          // R_lt values
-    const int nz   = 3 * BANK * nb;             // R entries of the tail in LDS
-    // FP64 inverses would spill the registers here: loaded after the restriction
-    T pv[BD];
-    if constexpr(sizeof(T) == 4)
-        bank_load(inv, b0 + (bi < nb ? bi : 0), pv);
-    const int above = (lt + 1 < L) ? lv.off[lt + 1] - base : span;
-    T         rl[kTailRPer];
-    int       upv[kTailSpanPer];
-    int       cbv[kTailSpanPer];
+    return (size_t)(3 * span + 3 * kFinThreads * levels) * sizeof(T)
+           + (size_t)kFinThreads * levels * sizeof(int) + (size_t)span * sizeof(unsigned);
+}
+
+// 16 bytes of T
+template <typename T>
+struct alignas(16) Vec16
+{
+    T v[16 / sizeof(T)];
+};
+
+// row `row` of bank gb's inverse (symmetric: the column the product needs)
+template <typename T>
+__device__ __forceinline__ void row_load(const T* __restrict__ inv, int gb, int row, T (&pv)[BD])
+{
+    constexpr int   W = 16 / sizeof(T);
+    const Vec16<T>* P = reinterpret_cast<const Vec16<T>*>(inv + (size_t)gb * BD * BD + row * BD);
 #pragma unroll
-    for(int h = 0; h < kTailRPer; h++)
+    for(int u = 0; u < BD / W; u++)
     {
-        const int i = threadIdx.x + h * kTailThreads;
-        rl[h]       = i < nr ? R[3 * (size_t)base + i] : (T)0;
-    }
+        Vec16<T> q = P[u];
 #pragma unroll
-    for(int h = 0; h < kTailSpanPer; h++)
-    {
-        const int i = threadIdx.x + h * kTailThreads;
-        upv[h]      = i < span ? going_next[base + i] : -1;
-        cbv[h]      = (i < span && i >= above) ? child_bank[base + i] - b0 : 0;
-    }
-#pragma unroll
-    for(int h = 0; h < kTailRPer; h++)
-    {
-        const int i = threadIdx.x + h * kTailThreads;
-        if(i < nz)
-            Rs[i] = rl[h];
-    }
-#pragma unroll
-    for(int h = 0; h < kTailSpanPer; h++)
-    {
-        const int i = threadIdx.x + h * kTailThreads;
-        if(i < span)
-        {
-            up[i] = upv[h];
-            if(i >= above)
-                cb[i] = (unsigned char)cbv[h];
-        }
-    }
-    __syncthreads();
-    for(int l = lt; l + 1 < L; l++)
-    {
-        const int e0 = lv.off[l] + lv.count[l], n1 = lv.off[l + 1];
-        for(int q = threadIdx.x; q < lv.count[l + 1]; q += blockDim.x)
-        {
-            const int p  = n1 + q;
-            const int gb = b0 + cb[p - base];
-            T         s0 = 0, s1 = 0, s2 = 0;
-            // the bank's parents and values read as batches of 8 members
-            // (reads past the level's end stay inside the tail's LDS rows;
-            // their values are not used), summed in node order
-#pragma unroll
-            for(int h = 0; h < BANK; h += 8)
-            {
-                int par[8];
-                T   v[24];
-#pragma unroll
-                for(int u = 0; u < 8; u++)
-                {
-                    const int g = gb * BANK + h + u;
-                    par[u]      = g < e0 ? up[g - base] : -1;
-                    v[3 * u]     = Rs[3 * (g - base)];
-                    v[3 * u + 1] = Rs[3 * (g - base) + 1];
-                    v[3 * u + 2] = Rs[3 * (g - base) + 2];
-                }
-#pragma unroll
-                for(int u = 0; u < 8; u++)
-                    if(par[u] == p)
-                    {
-                        s0 += v[3 * u];
-                        s1 += v[3 * u + 1];
-                        s2 += v[3 * u + 2];
-                    }
-            }
-            Rs[3 * (p - base)]     = s0;
-            Rs[3 * (p - base) + 1] = s1;
-            Rs[3 * (p - base) + 2] = s2;
-        }
-        __syncthreads();
-    }
-    if(bi < nb)
-    {
-        const int gb = b0 + bi;
-        const T*  rs = Rs + 3 * (gb * BANK - base);
-        if constexpr(sizeof(T) == 8)
-            bank_load(inv, gb, pv);
-        T z = 0;
-#pragma unroll
-        for(int u = 0; u < BD; u++)
-            z += pv[u] * rs[u];
-        Z[(size_t)gb * ZB + t] = z;
+        for(int k = 0; k < W; k++)
+            pv[u * W + k] = q.v[k];
     }
 }
 
-constexpr int kChainFast = 8;  // hierarchies up to 9 levels take an unrolled gather
-
-// z_v = Z[slot(v)] + sum_l Z[chain_l(v)];  r.z into a slot set; workgroup 0
-// clears two slot sets for later iterations.  NL = L - 1 chain entries per
-// node, known at compile time for NL <= kChainFast (every chain id is
-// loaded, then every gather issued: two memory round trips instead of two
-// per level; same summation order), or -1 for a runtime count.
-template <typename T, typename V, int NL>
-__global__ void __launch_bounds__(256)
-    k_mas_collect(int nv, int L, const int* __restrict__ slot_of, const int* __restrict__ chain,
-                  const T* __restrict__ Z, const V* __restrict__ r, V* __restrict__ z,
-                  double* rz_out, double* zero0, double* zero1,
-                  const int* __restrict__ done)
+template <typename T>
+__device__ __forceinline__ T row_product(const T (&pv)[BD], const T* rs)
 {
-    if(done && *done)
-        return;
-    int    v = (int)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    double d = 0.0;
-    if(v < nv)
+    T z = 0;
+#pragma unroll
+    for(int u = 0; u < BD; u++)
+        z += pv[u] * rs[u];
+    return z;
+}
+
+// z_v = Z[slot(v)] + sum_l z_l[chain_l(v)];  r.z into a slot set; workgroup 0
+// clears two slot sets for later iterations.  NL = L - 1 coarse levels.
+template <typename T, typename V, int NL>
+__global__ void __launch_bounds__(kFinThreads)
+    k_mas_finish(int nv, TailPlan tp, const int* __restrict__ slot_of,
+                 const int* __restrict__ chain, const int* __restrict__ child_bank,
+                 const unsigned* __restrict__ child_mask, const T* __restrict__ inv,
+                 const T* __restrict__ R, const T* __restrict__ Z, const V* __restrict__ r,
+                 V* __restrict__ z, double* rz_out, double* zero0, double* zero1,
+                 const int* __restrict__ done)
+{
+    // read with the first loads; a stopped solve leaves before it writes
+    const int     stop = done ? *done : 0;
+    constexpr int L  = NL + 1;
+    constexpr int NA = NL > 0 ? NL : 1;
+    extern __shared__ __align__(16) unsigned char fin_lds[];
+    __shared__ int wcnt[NA][kFinThreads / 64];
+    const int  tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int  ntl = L - tp.lt;  // tail levels
+    T*         Rs   = reinterpret_cast<T*>(fin_lds);
+    T*         zb   = Rs + 3 * tp.span;
+    int*       list = reinterpret_cast<int*>(zb + 3 * kFinThreads * ntl);
+    unsigned*  memb = reinterpret_cast<unsigned*>(list + kFinThreads * ntl);
+    const int  v    = (int)xcd_block(blockIdx.x, gridDim.x) * kFinThreads + tid;
+    const bool live = v < nv;
+    int        sl   = 0, g[NA];
+    double     r0 = 0.0, r1 = 0.0, r2 = 0.0;
+#pragma unroll
+    for(int l = 0; l < NL; l++)
+        g[l] = live ? chain[(size_t)v * NL + l] : -1;
+    if(live)
     {
-        int        s  = slot_of[v];
-        const T*   zs = Z + (size_t)(s >> 4) * ZB + 3 * (s & 15);
-        const int* ch = chain + (size_t)v * (L - 1);
-        T          z0, z1, z2;
-        double     r0 = 0.0, r1 = 0.0, r2 = 0.0;  // loaded with the ids, not after the stores
+        sl = slot_of[v];
         if(rz_out)
         {
             r0 = (double)r[3 * (size_t)v];
             r1 = (double)r[3 * (size_t)v + 1];
             r2 = (double)r[3 * (size_t)v + 2];
         }
-        if constexpr(NL >= 0)
+    }
+    const int b0 = tp.base / BANK;
+    int       fl[NA] = {};   // this vertex's tail nodes in the workgroup's list
+    int       total = 0;     // nodes in the list
+    T         pv[BD];
+    if(ntl > 0)
+    {
+        // R_lt (its padding is zero in memory too), four loads in flight per
+        // thread; zeros above it
+        constexpr int   W   = 16 / sizeof(T);
+        const int       n0  = 3 * tp.first, nv0 = n0 / W;
+        const Vec16<T>* src = reinterpret_cast<const Vec16<T>*>(R + 3 * (size_t)tp.base);
+        Vec16<T>*       dst = reinterpret_cast<Vec16<T>*>(Rs);
+        const int       mi  = tp.first + tid;  // the members of the levels above
+        unsigned        mb = 0, mm = 0;
+        if(mi < tp.span)
         {
-            int g[NL > 0 ? NL : 1];
+            mb = (unsigned)(child_bank[tp.base + mi] - b0) << 16;
+            mm = child_mask[tp.base + mi];
+        }
+        for(int i = tid; i < nv0; i += 4 * kFinThreads)
+        {
+            Vec16<T> q[4];
 #pragma unroll
-            for(int l = 0; l < NL; l++)
-                g[l] = ch[l];
-            z0 = zs[0];
-            z1 = zs[1];
-            z2 = zs[2];
-            T zz[NL > 0 ? NL : 1][3];
-#pragma unroll
-            for(int l = 0; l < NL; l++)
+            for(int k = 0; k < 4; k++)
             {
-                const T* zg = Z + (size_t)(g[l] >> 4) * ZB + 3 * (g[l] & 15);
-                zz[l][0]    = zg[0];
-                zz[l][1]    = zg[1];
-                zz[l][2]    = zg[2];
+                const int j = i + k * kFinThreads;
+                q[k]        = src[j < nv0 ? j : i];
             }
 #pragma unroll
-            for(int l = 0; l < NL; l++)
+            for(int k = 0; k < 4; k++)
             {
-                z0 += zz[l][0];
-                z1 += zz[l][1];
-                z2 += zz[l][2];
+                const int j = i + k * kFinThreads;
+                if(j < nv0)
+                    dst[j] = q[k];
             }
         }
-        else
-        {
-            z0 = zs[0];
-            z1 = zs[1];
-            z2 = zs[2];
-            for(int l = 0; l < L - 1; l++)
+        for(int i = n0 + tid; i < 3 * tp.span; i += kFinThreads)
+            Rs[i] = (T)0;
+        if(mi < tp.span)
+            memb[mi] = mb | mm;
+        for(int i = mi + kFinThreads; i < tp.span; i += kFinThreads)
+            memb[i] = ((unsigned)(child_bank[tp.base + i] - b0) << 16) | child_mask[tp.base + i];
+        // distinct tail nodes: the heads of runs of equal nodes along the
+        // vertices of a wave (a run that crosses waves is listed twice)
+        int rank[NA];
+#pragma unroll
+        for(int l = 0; l < NL; l++)
+            if(l + 1 >= tp.lt)
             {
-                const T* zg = Z + (size_t)(ch[l] >> 4) * ZB + 3 * (ch[l] & 15);
-                z0 += zg[0];
-                z1 += zg[1];
-                z2 += zg[2];
+                const int  up   = __shfl_up(g[l], 1, 64);
+                const bool head = live && (lane == 0 || up != g[l]);
+                const unsigned long long m = __ballot(head);
+                rank[l] = __popcll(m & ((2ull << lane) - 1ull)) - 1;
+                if(lane == 0)
+                    wcnt[l][w] = __popcll(m);
+                fl[l] = head ? 1 : 0;
             }
+        if(stop)
+            return;
+        __syncthreads();
+#pragma unroll
+        for(int l = 0; l < NL; l++)
+            if(l + 1 >= tp.lt)
+            {
+                int at = total;
+#pragma unroll
+                for(int q = 0; q < kFinThreads / 64; q++)
+                {
+                    const int c = wcnt[l][q];
+                    at += q < w ? c : 0;
+                    total += c;
+                }
+                const bool head = fl[l] != 0;
+                fl[l]           = at + rank[l];
+                if(head)
+                    list[fl[l]] = g[l] - tp.base;
+            }
+        __syncthreads();
+        // the first product's row is requested before the restriction
+        if(tid < 3 * total)
+        {
+            const int n = list[tid / 3];
+            row_load(inv, b0 + n / BANK, 3 * (n % BANK) + tid % 3, pv);
+        }
+    }
+    if(stop)
+        return;
+    T z0 = 0, z1 = 0, z2 = 0;
+    T zz0[NA] = {}, zz1[NA] = {}, zz2[NA] = {};
+    if(live)
+    {
+        const T* zs = Z + (size_t)(sl >> 4) * ZB + 3 * (sl & 15);
+        z0          = zs[0];
+        z1          = zs[1];
+        z2          = zs[2];
+#pragma unroll
+        for(int l = 0; l < NL; l++)
+            if(l + 1 < tp.lt)
+            {
+                const T* zg = Z + (size_t)(g[l] >> 4) * ZB + 3 * (g[l] & 15);
+                zz0[l]      = zg[0];
+                zz1[l]      = zg[1];
+                zz2[l]      = zg[2];
+            }
+    }
+    if(ntl > 0)
+    {
+#pragma unroll
+        for(int l = 1; l < NL; l++)  // level l to level l + 1
+            if(l >= tp.lt)
+            {
+                const int o = tp.off[l + 1] - tp.base;
+                for(int q = tid; q < 3 * tp.count[l + 1]; q += kFinThreads)
+                {
+                    const unsigned mk = memb[o + q / 3];
+                    const T*       rs = Rs + 3 * BANK * (mk >> 16) + q % 3;
+                    T              m[BANK], s = 0;
+#pragma unroll
+                    for(int u = 0; u < BANK; u++)
+                        m[u] = rs[3 * u];
+#pragma unroll
+                    for(int u = 0; u < BANK; u++)
+                        s = (mk >> u) & 1u ? s + m[u] : s;
+                    Rs[3 * o + q] = s;
+                }
+                __syncthreads();
+            }
+        for(int f = tid; f < 3 * total; f += kFinThreads)
+        {
+            const int n = list[f / 3];
+            if(f >= kFinThreads)
+                row_load(inv, b0 + n / BANK, 3 * (n % BANK) + f % 3, pv);
+            zb[f] = row_product(pv, Rs + 3 * BANK * (n / BANK));
+        }
+        __syncthreads();
+    }
+    double d = 0.0;
+    if(live)
+    {
+#pragma unroll
+        for(int l = 0; l < NL; l++)
+        {
+            const bool tail = l + 1 >= tp.lt;
+            const int  o    = tail ? 3 * fl[l] : 0;
+            const T    t0 = zb[o], t1 = zb[o + 1], t2 = zb[o + 2];
+            z0 += tail ? t0 : zz0[l];
+            z1 += tail ? t1 : zz1[l];
+            z2 += tail ? t2 : zz2[l];
         }
         z[3 * (size_t)v]     = (V)z0;
         z[3 * (size_t)v + 1] = (V)z1;
@@ -873,9 +927,9 @@ __global__ void __launch_bounds__(256)
     if(blockIdx.x == 0)
     {
         if(zero0)
-            slot_set_clear(zero0, threadIdx.x);
+            slot_set_clear(zero0, tid);
         if(zero1)
-            slot_set_clear(zero1, threadIdx.x);
+            slot_set_clear(zero1, tid);
     }
 }
 
@@ -941,6 +995,7 @@ void Mas::init(const Bsr& A, const int* part_id, const MasConfig& cfg, hipStream
     size_t bound = (size_t)L_ * (total_map_ + BANK) + BANK;
     going_next_.resize(bound);
     child_bank_.resize(bound);
+    child_mask_.resize(bound);
     bank_first_.resize(bound / BANK + 1);
     bank_ncl_.resize(bound / BANK + 1);
     std::vector<int> lvl0(2 * (L_ + 2), 0);
@@ -962,7 +1017,7 @@ void Mas::cluster_level(int level, hipStream_t s)
     hipLaunchKernelGGL(k_assign, dim3(g), dim3(256), 0, s, level, total_map_, lvl_.data(),
                        vert_of_slot_.data(), comp_.data(), bank_prefix_.data(), bank_cnt_.data(),
                        newid_.data(), going_next_.data(), bank_first_.data(), bank_ncl_.data(),
-                       child_bank_.data());
+                       child_bank_.data(), child_mask_.data());
     SG_LAUNCH_CHECK();
     if(level + 1 <= L_ - 1)
     {
@@ -1100,90 +1155,75 @@ void Mas::invert(hipStream_t s)
     SG_LAUNCH_CHECK();
 }
 
-template <typename T, typename V>
-static void mas_apply_t(Profiler* prof, int nparts, int L, int nv, const std::vector<int>& lvl,
-                        const int* vert_of_slot, const int* slot_of, const int* chain,
-                        const int* going_next, const int* bank_first, const int* bank_ncl,
-                        const int* child_bank, const T* inv, T* R, T* Z, V* x, V* r, const V* p,
-                        const V* Ap, const double* rz_prev, const double* pap, V* z,
-                        double* rz_out, double* zero0, double* zero1, const int* done,
-                        hipStream_t s, bool defer_rz)
+// the first level whose tail fits k_mas_finish's LDS; the levels below it get
+// launches of their own.  64 KB: two workgroups per CU.  Starting one level
+// later than it fits costs its launch (46,656 rows, FP32: 38.7 us per PCG
+// iteration with the tail at level 2, 45.0 at level 4; 173,225 rows: 104.4 at
+// level 2, 107.9 at level 3).
+template <typename T>
+static TailPlan tail_plan(int L, const std::vector<int>& lvl)
 {
-    // Plan: separate launches for levels 1 .. lt-1 (each stores the next
-    // level's R), then one k_mas_coarse launch for the tail lt .. L-1, whose
-    // workgroups load R_lt and restrict the levels above in LDS.  (Summing R_lt
-    // from level lt-1 inside the tail launch costs two dependent gathers,
-    // more than the extra launch.)
-    int lt = L;
-    if(L > 1)
+    TailPlan tp;
+    for(int q = 0; q < L; q++)
     {
-        for(int l = 1; l < L; l++)
-        {
-            int nbk  = (lvl[2 * l] + BANK - 1) / BANK;
-            int span = lvl[2 * (L - 1) + 1] + lvl[2 * (L - 1)] - lvl[2 * l + 1];
-            if(nbk <= kTailBanks && span <= kTailNodes)
-            {
-                lt = l;
-                break;
-            }
-        }
+        tp.count[q] = lvl[2 * q];
+        tp.off[q]   = lvl[2 * q + 1];
     }
+    for(tp.lt = 1; tp.lt < L; tp.lt++)
+    {
+        tp.base  = tp.off[tp.lt];
+        tp.first = (tp.count[tp.lt] + BANK - 1) / BANK * BANK;
+        tp.span = (tp.off[L - 1] + tp.count[L - 1] - tp.base + BANK - 1) / BANK * BANK;
+        if(finish_lds<T>(tp.span, L - tp.lt) <= (size_t)kFinLds)
+            return tp;
+    }
+    tp.base = tp.span = 0;
+    return tp;
+}
+
+template <typename T, typename V>
+void Mas::apply_levels(const T* inv, T* R, T* Z, V* x, V* r, const V* p, const V* Ap,
+                       const double* rz_prev, const double* pap, V* z, double* rz_out,
+                       double* zero0, double* zero1, const int* done, hipStream_t s,
+                       bool defer_rz)
+{
+    SG_CHECK(grid_for(nv_, kFinThreads) <= (unsigned)kSetMaxBlocks, SGIPC_ECAPACITY,
+             "MAS: system too large for the fixed-order reductions");
     auto ev = prof ? prof->kernel_events("mas_apply_l0")
                    : std::pair<hipEvent_t, hipEvent_t>{nullptr, nullptr};
-    hipExtLaunchKernelGGL((k_mas_l0<T, V>), dim3(nparts), dim3(64), 0, s, ev.first, ev.second, 0,
-                          vert_of_slot, x, r, p, Ap, rz_prev, pap, inv, going_next, bank_first,
-                          bank_ncl, R, Z, L > 1 ? 1 : 0, done);
+    hipExtLaunchKernelGGL((k_mas_l0<T, V>), dim3(nparts_), dim3(64), 0, s, ev.first, ev.second, 0,
+                          vert_of_slot_.data(), x, r, p, Ap, rz_prev, pap, inv,
+                          going_next_.data(), bank_first_.data(), bank_ncl_.data(), R, Z,
+                          L_ > 1 ? 1 : 0, done);
     SG_LAUNCH_CHECK();
-    if(L > 1)
+    const TailPlan tp = tail_plan<T>(L_, h_lvl_);
+    for(int l = 1; l < tp.lt && l < L_; l++)
     {
-        for(int l = 1; l < lt; l++)
-        {
-            int count = lvl[2 * l], off = lvl[2 * l + 1];
-            int nbk   = (count + BANK - 1) / BANK;
-            hipLaunchKernelGGL(k_mas_lx<T>, dim3(nbk), dim3(64), 0, s, off / BANK, off, count, inv,
-                               going_next, bank_first, bank_ncl, R, Z, l + 1 < L ? 1 : 0, done);
-            SG_LAUNCH_CHECK();
-        }
-        SG_CHECK(L <= 24, -1, "MAS: more than 24 levels");
-        LevelTable lv{};
-        for(int q = 0; q < L; q++)
-        {
-            lv.count[q] = lvl[2 * q];
-            lv.off[q]   = lvl[2 * q + 1];
-        }
-        if(lt < L)
-        {
-            int span = lvl[2 * (L - 1) + 1] + lvl[2 * (L - 1)] - lvl[2 * lt + 1];
-            int nbt  = (span + BANK - 1) / BANK;
-            int ntw  = (nbt + kCoarseWaves - 1) / kCoarseWaves;
-            hipLaunchKernelGGL(k_mas_coarse<T>, dim3(ntw), dim3(kTailThreads), 0, s, lv, L, lt,
-                               inv, going_next, child_bank, R, Z, done);
-            SG_LAUNCH_CHECK();
-        }
+        int nbk = (tp.count[l] + BANK - 1) / BANK;
+        hipLaunchKernelGGL(k_mas_lx<T>, dim3(nbk), dim3(64), 0, s, tp.off[l] / BANK, tp.off[l],
+                           tp.count[l], inv, going_next_.data(), bank_first_.data(),
+                           bank_ncl_.data(), R, Z, l + 1 < L_ ? 1 : 0, done);
+        SG_LAUNCH_CHECK();
     }
-    SG_CHECK(grid_for(nv, 256) <= (unsigned)kSetMaxBlocks, SGIPC_ECAPACITY,
-             "MAS: system too large for the fixed-order reductions");
-    auto collect = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3(grid_for(nv, 256)), dim3(256), 0, s, nv, L, slot_of, chain,
-                           Z, r, z, rz_out, zero0, zero1, done);
+    auto finish = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(grid_for(nv_, kFinThreads)), dim3(kFinThreads),
+                           tp.lt < L_ ? finish_lds<T>(tp.span, L_ - tp.lt) : 64, s, nv_, tp,
+                           slot_of_.data(), chain_.data(), child_bank_.data(),
+                           child_mask_.data(), inv, R, Z, r, z, rz_out, zero0, zero1, done);
     };
-    static_assert(kChainFast == 8, "collect dispatch below covers NL = 0 .. 8");
-    switch(L - 1)
+    static_assert(kMaxLevels == 6, "the dispatch below covers 1 .. 6 levels");
+    switch(L_)
     {
-    case 0: collect(k_mas_collect<T, V, 0>); break;
-    case 1: collect(k_mas_collect<T, V, 1>); break;
-    case 2: collect(k_mas_collect<T, V, 2>); break;
-    case 3: collect(k_mas_collect<T, V, 3>); break;
-    case 4: collect(k_mas_collect<T, V, 4>); break;
-    case 5: collect(k_mas_collect<T, V, 5>); break;
-    case 6: collect(k_mas_collect<T, V, 6>); break;
-    case 7: collect(k_mas_collect<T, V, 7>); break;
-    case 8: collect(k_mas_collect<T, V, 8>); break;
-    default: collect(k_mas_collect<T, V, -1>); break;
+    case 1: finish(k_mas_finish<T, V, 0>); break;
+    case 2: finish(k_mas_finish<T, V, 1>); break;
+    case 3: finish(k_mas_finish<T, V, 2>); break;
+    case 4: finish(k_mas_finish<T, V, 3>); break;
+    case 5: finish(k_mas_finish<T, V, 4>); break;
+    default: finish(k_mas_finish<T, V, 5>); break;
     }
     SG_LAUNCH_CHECK();
     if(rz_out && !defer_rz)
-        set_finalize(rz_out, (int)grid_for(nv, 256), done, s);
+        set_finalize(rz_out, (int)grid_for(nv_, kFinThreads), done, s);
 }
 
 template <typename V>
@@ -1193,19 +1233,11 @@ void Mas::apply_fused_t(V* x, V* r, const V* p, const V* Ap, const double* rz_pr
 {
     SG_CHECK(built_, -5, "MAS apply before build");
     if(cfg_.fp32)
-        mas_apply_t<float, V>(prof, nparts_, L_, nv_, h_lvl_, vert_of_slot_.data(),
-                              slot_of_.data(), chain_.data(), going_next_.data(),
-                              bank_first_.data(), bank_ncl_.data(), child_bank_.data(),
-                              inv32_.data(), R32_.data(),
-                              Z32_.data(), x, r, p, Ap, rz_prev, pap, z, rz_out, zero0, zero1,
-                              done, s, defer_rz);
+        apply_levels<float, V>(inv32_.data(), R32_.data(), Z32_.data(), x, r, p, Ap, rz_prev, pap,
+                               z, rz_out, zero0, zero1, done, s, defer_rz);
     else
-        mas_apply_t<double, V>(prof, nparts_, L_, nv_, h_lvl_, vert_of_slot_.data(),
-                               slot_of_.data(), chain_.data(), going_next_.data(),
-                               bank_first_.data(), bank_ncl_.data(), child_bank_.data(),
-                               inv64_.data(), R64_.data(),
-                               Z64_.data(), x, r, p, Ap, rz_prev, pap, z, rz_out, zero0, zero1,
-                               done, s, defer_rz);
+        apply_levels<double, V>(inv64_.data(), R64_.data(), Z64_.data(), x, r, p, Ap, rz_prev,
+                                pap, z, rz_out, zero0, zero1, done, s, defer_rz);
 }
 
 void Mas::apply_fused(double* x, double* r, const double* p, const double* Ap,

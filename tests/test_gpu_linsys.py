@@ -209,3 +209,33 @@ def test_mas_bank_inverse_bit_exact(systems, oracle, name, prec):
         assert np.array_equal(inv.view(np.uint64), expect.view(np.uint64)), f"bank {b}"
         checked += 1
     assert checked == nbank > 0
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("kind", ["chain", "diagonal"])
+@pytest.mark.parametrize("nb", [1, 17, 255, 257, 1000])
+def test_mas_apply_workgroup_edges(oracle, nb, kind, prec):
+    """Systems that end inside, at and after a 256-vertex workgroup of the
+    apply's last launch.  A chain has one tail node per bank; without
+    couplings every vertex is its own node on every level, so a workgroup
+    multiplies more rows than it has threads."""
+    import sgipc
+    rng = np.random.default_rng(nb)
+    n = np.arange(nb)
+    S = rng.normal(size=(nb, 3, 3))
+    vals = 4.0 * np.eye(3) + 0.3 * (S + S.transpose(0, 2, 1))
+    rows, cols = n, n
+    if kind == "chain" and nb > 1:
+        off = 0.4 * rng.normal(size=(nb - 1, 3, 3))
+        vals = np.concatenate([vals + 2.0 * np.eye(3), off])
+        rows, cols = np.concatenate([n, n[:-1]]), np.concatenate([n, n[1:]])
+    A = oracle.bsr_from_upper_triplets(nb, rows, cols, vals.reshape(-1, 9))
+    part = (n // 16).astype(np.int32)
+    fp32 = prec == "fp32"
+    ls = sgipc.LinearSystem(A.rowptr, A.cols, A.vals, part, sgipc.SGIPC_PRECOND_MAS,
+                            sgipc.SGIPC_MAS_FP32 if fp32 else sgipc.SGIPC_MAS_FP64)
+    m = oracle.Mas(A, part, fp32=fp32)
+    np.testing.assert_array_equal(ls.mas_info()[1], m.level_sizes())
+    r = rng.normal(size=3 * nb)
+    # FP32: inverses and sums of 48 products per level round at 6e-8 each
+    assert rel(ls.precond(r), m.apply(r)) < (2e-5 if fp32 else 1e-10)
