@@ -5,6 +5,7 @@
 #include <string>
 
 #include "linsys.h"
+#include "persist.h"
 #include "sgipc.h"
 
 namespace sgipc
@@ -47,6 +48,7 @@ struct sgipc_linear_system
     int                  dev     = 0;  // device current at creation
     sgipc::Bsr           A;
     sgipc::Mas           mas;
+    sgipc::PersistPlan   plan;
     sgipc::Pcg           pcg;
     sgipc::Pcg           pcg_na;       // solver of sgipc_ls_pcg_noalloc (no memory of its own)
     int                  precond = 1;

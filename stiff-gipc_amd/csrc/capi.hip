@@ -71,6 +71,10 @@ int sgipc_ls_create(int32_t nb, int32_t nnzb, const int32_t* rowptr, const int32
             }
             else
                 ls->pcg.build_diag(ls->A, ls->s);
+            ls->plan.build(ls->A,
+                           precond == SGIPC_PRECOND_MAS ? ls->mas.part_first()
+                                                        : std::vector<int>(),
+                           ls->s);
             SG_HIP(hipStreamSynchronize(ls->s));
         }
         catch(...)
@@ -244,7 +248,7 @@ int sgipc_ls_pcg(sgipc_ls_t ls, const double* b, double* x, const sgipc_pcg_cfg*
         SG_HIP(hipEventCreate(&e0));
         SG_HIP(hipEventCreate(&e1));
         SG_HIP(hipEventRecord(e0, ls->s));
-        PcgStats st = ls->pcg.solve(SysView{&ls->A, nullptr},
+        PcgStats st = ls->pcg.solve(SysView{&ls->A, nullptr, &ls->plan},
                                     ls->precond == SGIPC_PRECOND_MAS ? Precond::Mas : Precond::Diag,
                                     &ls->mas, ls->b.data(), ls->x.data(), pc, ls->s);
         SG_HIP(hipEventRecord(e1, ls->s));

@@ -5,6 +5,7 @@
 #include "../../include/sgipc.h"
 #include "learned.h"
 #include "linsys.h"
+#include "persist.h"
 #include "sim_kernels.h"
 
 namespace sgipc
@@ -172,6 +173,7 @@ class Context
     Bsr   A_;
     Coo   coo_;
     Mas   mas_;
+    PersistPlan plan_;
     Pcg   pcg_;
     Lbvh  bf_, be_;
     SimDev dev_;

@@ -739,6 +739,8 @@ Context::Context(const sgipc_scene_desc& d)
                 npart[nfem_ + 4 * b + k] = maxp + 1 + b;
         mas_.init(A_, npart.data(), mc, s_);
     }
+    plan_.build(A_,
+                d.precond == SGIPC_PRECOND_MAS ? mas_.part_first() : std::vector<int>(), s_);
     mas_.prof = &prof_;
     pcg_.prof = &prof_;
     // block-Jacobi mode: each affine body's 12x12 block as one block
@@ -1239,7 +1241,7 @@ void Context::newton_iteration(sgipc_iter_stats* st)
         mm_write_system(A_path, b_path, nn_, rp, cl, vl, g);
     }
     // ---- linear solve
-    SysView S{&A_, &coo_};
+    SysView S{&A_, &coo_, &plan_};
     Precond pc = desc_.precond == SGIPC_PRECOND_MAS ? Precond::Mas : Precond::Diag;
     if(pc == Precond::Mas)
         mas_.build(S, s_);

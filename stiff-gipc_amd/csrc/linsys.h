@@ -84,11 +84,15 @@ struct Coo
     void ensure_entries(int n);
 };
 
+class PersistPlan;  // persist.h
+
 // view of A = static BSR + COO tail
 struct SysView
 {
     const Bsr* A   = nullptr;
     const Coo* coo = nullptr;  // may be null; its row-sorted copy must be current
+    // may be null: the plan of the one-launch solve of this pattern
+    PersistPlan* plan = nullptr;
 };
 
 // ------------------------------------------------------------ reductions
@@ -154,6 +158,16 @@ class MasGalerkin
     DBuf<double>   eb_[2];
 };
 
+// device pointers of a built hierarchy, T: precision of the inverses
+template <typename T>
+struct MasView
+{
+    const int *     vert_of_slot, *going_next, *bank_first, *bank_ncl, *chain, *child_bank;
+    const unsigned* child_mask;
+    const T*        inv;
+    T *             R, *Z;
+};
+
 class Mas
 {
   public:
@@ -185,6 +199,11 @@ class Mas
     // workgroups of the apply's last launch (partials of its rz set)
     int collect_blocks() const { return (int)grid_for(nv_, 256); }
 
+    template <typename T>
+    MasView<T> view();
+    bool       fp32() const { return cfg_.fp32; }
+    // first row of each part (size parts + 1)
+    const std::vector<int>& part_first() const { return part_first_; }
     int levels() const { return L_; }
     int total_clusters() const { return total_clusters_; }
     const std::vector<int>& level_sizes() const { return h_lvl_; }  // (count, off) pairs
@@ -215,6 +234,7 @@ class Mas
     MasConfig cfg_;
     int       nv_ = 0, nparts_ = 0, total_map_ = 0, L_ = 0, total_clusters_ = 0;
     bool      built_ = false;
+    std::vector<int> part_first_;
     DBuf<int>      slot_of_, vert_of_slot_;
     DBuf<unsigned> mask0_static_;
     DBuf<int>      xa_, xb_;   // static cross-bank edges (unordered)
@@ -301,6 +321,11 @@ enum class Precond
     Diag = 0,
     Mas  = 1
 };
+
+template <>
+MasView<float> Mas::view<float>();
+template <>
+MasView<double> Mas::view<double>();
 
 class Pcg
 {

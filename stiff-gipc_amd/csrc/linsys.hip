@@ -8,7 +8,7 @@
 // scalar stays on the device: pAp[k] and rz[k] are summed in a fixed order
 // into slot sets (common.h) and the consuming kernels derive a and b from
 // them; the host reads back only at the convergence test.
-#include "linsys.h"
+#include "persist.h"
 
 #include "../../include/sgipc.h"
 
@@ -1067,6 +1067,30 @@ PcgStats Pcg::solve_t(const SysView& S, Precond pc, Mas* mas, const V* b, V* x,
     PcgVecs<V>& W     = vecs<V>();
     ensure(n);
     W.ensure(n);
+    if constexpr(sizeof(V) == sizeof(double))
+        if(!b64 && S.plan && S.plan->ready() && (pc == Precond::Mas || nbody_ == 0))
+        {
+            // the whole solve in one launch (persist.hip)
+            if(pc == Precond::Diag)
+                build_diag(*S.A, s);
+            PersistResult pr;
+            if(persist_solve(*S.plan, S, pc == Precond::Mas ? mas : nullptr, dinv_.data(), b, x,
+                             W.z.data(), W.p[0].data(), W.p[1].data(), cfg, maxit, every, &pr, s))
+            {
+                PcgStats st;
+                st.rz0 = pr.rz0;
+                if(pr.rz0 == 0.0 || !(pr.rz0 == pr.rz0))
+                {
+                    st.converged = (pr.rz0 == 0.0);
+                    return st;
+                }
+                SG_CHECK(pr.bad == 0, -4, "PCG breakdown: non-finite r.z");
+                st.rz         = pr.rz;
+                st.converged  = pr.stop_at != 0;
+                st.iterations = pr.stop_at != 0 ? pr.stop_at : maxit;
+                return st;
+            }
+        }
     SG_HIP(hipMemsetAsync(red_.data(), 0, red_.size() * sizeof(double), s));
     SG_HIP(hipMemsetAsync(ctl_.data(), 0, ctl_.size() * sizeof(int), s));
     SG_HIP(hipMemsetAsync(ctl_d_.data(), 0, ctl_d_.size() * sizeof(double), s));

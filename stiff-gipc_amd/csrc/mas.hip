@@ -23,15 +23,13 @@
 // The apply is level-synchronous and atomic-free: every node of level l+1 lies
 // inside a single bank of level l, so restriction is a bank-local LDS
 // reduction done by the same wave that applies that bank's inverse.
-#include "linsys.h"
+#include "mas_tail.h"
 #include "sgipc.h"
+
+#include <algorithm>
 
 namespace sgipc
 {
-
-constexpr int BANK = 16;
-constexpr int BD   = 48;  // 3 * BANK
-constexpr int ZB   = 64;  // Z entries per bank: one per lane, lanes 48..63 padding
 
 static int compute_num_levels(int nv)
 {
@@ -318,16 +316,6 @@ __global__ void __launch_bounds__(256) k_mas_gather(int nnz, const int* __restri
             M[a * BD + c] = blk[3 * a + c];
 }
 
-// Ordering of LDS between the lanes of a single-wave workgroup: the LDS
-// instructions of one wave execute in program order, so a compiler-only
-// wave barrier suffices; __syncthreads would also make the wave wait for its
-// outstanding global stores (workgroup-scope release).
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_wave_barrier();
-}
-
-
 // One wave per bank: load 48x48 into LDS, zero diagonal -> 1, in-place
 // Gauss-Jordan without pivoting (bank matrices are SPD), blocked by 16x16
 // tiles so that three quarters of the work runs on FP64 MFMA.  Eliminating
@@ -481,23 +469,6 @@ __global__ void __launch_bounds__(64) k_mas_invert(const double* __restrict__ B,
 }
 
 // ---------------------------------------------------------------- apply
-// One bank's product z = Binv R with one wave: lane u < 48 holds R_u, lane
-// t < 48 produces z_t (lanes 48..63 compute a copy of lane 0's and store it
-// into the bank's padding).  The 48 entries a lane needs (column t of the
-// stored transpose) are loaded before the products so their latencies
-// overlap; every lane stores unconditionally so the compiler keeps the loads
-// together instead of sinking them into a guarded block.
-template <typename T>
-__device__ __forceinline__ void bank_load(const T* __restrict__ inv, int gb, T (&pv)[BD])
-{
-    const int t  = __lane_id();
-    const int tc = t < BD ? t : 0;
-    const T*  P  = inv + (size_t)gb * BD * BD + tc;
-#pragma unroll
-    for(int u = 0; u < BD; u++)
-        pv[u] = P[u * BD];
-}
-
 template <typename T>
 __device__ __forceinline__ T bank_apply(const T (&pv)[BD], T rv)
 {
@@ -672,18 +643,7 @@ __global__ void __launch_bounds__(64) k_mas_lx(int bank0, int node0, int count,
 // PCG iteration 33.2 to 25.7 us on 6,480 rows (FP64 MAS), 41.3 to 38.4 us on
 // 46,656 rows, 106.8 to 102.3 us on 173,225 rows.
 constexpr int kFinThreads = 256;
-constexpr int kMaxLevels  = 6;          // compute_num_levels' bound
 constexpr int kFinLds     = 64 * 1024;  // LDS of one workgroup at most (two per CU)
-struct TailPlan
-{
-    int lt    = 0;  // first tail level (L: no tail)
-    int base  = 0;  // global id of the tail's first node (a multiple of 16)
-    int span  = 0;  // padded nodes of the tail
-    int first = 0;  // padded nodes of level lt
-    int count[kMaxLevels] = {};
-    int off[kMaxLevels]   = {};
-};
-
 // LDS of k_mas_finish: R of the tail, the products of the distinct tail nodes
 // (three components per node, at most kFinThreads nodes per level), their
 // list, the members of the nodes above lt
@@ -692,39 +652,6 @@ static size_t finish_lds(int span, int levels)
 {
     return (size_t)(3 * span + 3 * kFinThreads * levels) * sizeof(T)
            + (size_t)kFinThreads * levels * sizeof(int) + (size_t)span * sizeof(unsigned);
-}
-
-// 16 bytes of T
-template <typename T>
-struct alignas(16) Vec16
-{
-    T v[16 / sizeof(T)];
-};
-
-// row `row` of bank gb's inverse (symmetric: the column the product needs)
-template <typename T>
-__device__ __forceinline__ void row_load(const T* __restrict__ inv, int gb, int row, T (&pv)[BD])
-{
-    constexpr int   W = 16 / sizeof(T);
-    const Vec16<T>* P = reinterpret_cast<const Vec16<T>*>(inv + (size_t)gb * BD * BD + row * BD);
-#pragma unroll
-    for(int u = 0; u < BD / W; u++)
-    {
-        Vec16<T> q = P[u];
-#pragma unroll
-        for(int k = 0; k < W; k++)
-            pv[u * W + k] = q.v[k];
-    }
-}
-
-template <typename T>
-__device__ __forceinline__ T row_product(const T (&pv)[BD], const T* rs)
-{
-    T z = 0;
-#pragma unroll
-    for(int u = 0; u < BD; u++)
-        z += pv[u] * rs[u];
-    return z;
 }
 
 // z_v = Z[slot(v)] + sum_l z_l[chain_l(v)];  r.z into a slot set; workgroup 0
@@ -882,15 +809,7 @@ __global__ void __launch_bounds__(kFinThreads)
                 for(int q = tid; q < 3 * tp.count[l + 1]; q += kFinThreads)
                 {
                     const unsigned mk = memb[o + q / 3];
-                    const T*       rs = Rs + 3 * BANK * (mk >> 16) + q % 3;
-                    T              m[BANK], s = 0;
-#pragma unroll
-                    for(int u = 0; u < BANK; u++)
-                        m[u] = rs[3 * u];
-#pragma unroll
-                    for(int u = 0; u < BANK; u++)
-                        s = (mk >> u) & 1u ? s + m[u] : s;
-                    Rs[3 * o + q] = s;
+                    Rs[3 * o + q] = member_sum(Rs + 3 * BANK * (mk >> 16), mk, q % 3);
                 }
                 __syncthreads();
             }
@@ -957,6 +876,11 @@ void Mas::init(const Bsr& A, const int* part_id, const MasConfig& cfg, hipStream
     }
     nparts_    = maxpart + 1;
     total_map_ = BANK * nparts_;
+    part_first_.assign(nparts_ + 1, nv_);
+    for(int v = nv_ - 1; v >= 0; v--)
+        part_first_[slot[v] / BANK] = v;
+    for(int q = nparts_ - 1; q >= 0; q--)  // empty parts start where the next one does
+        part_first_[q] = std::min(part_first_[q], part_first_[q + 1]);
     L_         = compute_num_levels(nv_);
     std::vector<int>      vos(total_map_, -1);
     std::vector<unsigned> m0(total_map_, 0u);
@@ -1160,27 +1084,6 @@ void Mas::invert(hipStream_t s)
 // later than it fits costs its launch (46,656 rows, FP32: 38.7 us per PCG
 // iteration with the tail at level 2, 45.0 at level 4; 173,225 rows: 104.4 at
 // level 2, 107.9 at level 3).
-template <typename T>
-static TailPlan tail_plan(int L, const std::vector<int>& lvl)
-{
-    TailPlan tp;
-    for(int q = 0; q < L; q++)
-    {
-        tp.count[q] = lvl[2 * q];
-        tp.off[q]   = lvl[2 * q + 1];
-    }
-    for(tp.lt = 1; tp.lt < L; tp.lt++)
-    {
-        tp.base  = tp.off[tp.lt];
-        tp.first = (tp.count[tp.lt] + BANK - 1) / BANK * BANK;
-        tp.span = (tp.off[L - 1] + tp.count[L - 1] - tp.base + BANK - 1) / BANK * BANK;
-        if(finish_lds<T>(tp.span, L - tp.lt) <= (size_t)kFinLds)
-            return tp;
-    }
-    tp.base = tp.span = 0;
-    return tp;
-}
-
 template <typename T, typename V>
 void Mas::apply_levels(const T* inv, T* R, T* Z, V* x, V* r, const V* p, const V* Ap,
                        const double* rz_prev, const double* pap, V* z, double* rz_out,
@@ -1196,7 +1099,9 @@ void Mas::apply_levels(const T* inv, T* R, T* Z, V* x, V* r, const V* p, const V
                           going_next_.data(), bank_first_.data(), bank_ncl_.data(), R, Z,
                           L_ > 1 ? 1 : 0, done);
     SG_LAUNCH_CHECK();
-    const TailPlan tp = tail_plan<T>(L_, h_lvl_);
+    const TailPlan tp = tail_plan(L_, h_lvl_, [](int span, int levels) {
+        return finish_lds<T>(span, levels) <= (size_t)kFinLds;
+    });
     for(int l = 1; l < tp.lt && l < L_; l++)
     {
         int nbk = (tp.count[l] + BANK - 1) / BANK;
@@ -1260,6 +1165,21 @@ void Mas::apply(const double* r, double* z, hipStream_t s)
 {
     apply_fused(nullptr, const_cast<double*>(r), nullptr, nullptr, nullptr, nullptr, z, nullptr,
                 nullptr, nullptr, nullptr, s);
+}
+
+template <>
+MasView<float> Mas::view<float>()
+{
+    return {vert_of_slot_.data(), going_next_.data(), bank_first_.data(), bank_ncl_.data(),
+            chain_.data(), child_bank_.data(), child_mask_.data(), inv32_.data(), R32_.data(),
+            Z32_.data()};
+}
+template <>
+MasView<double> Mas::view<double>()
+{
+    return {vert_of_slot_.data(), going_next_.data(), bank_first_.data(), bank_ncl_.data(),
+            chain_.data(), child_bank_.data(), child_mask_.data(), inv64_.data(), R64_.data(),
+            Z64_.data()};
 }
 
 std::vector<int> Mas::chain_host(hipStream_t s) const

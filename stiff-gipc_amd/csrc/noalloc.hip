@@ -94,7 +94,7 @@ int sgipc_ls_pcg_noalloc(sgipc_ls_t ls, const double* b, double* x, const sgipc_
         pc.mixed       = false;
         auto t0        = std::chrono::steady_clock::now();
         SG_HIP(hipMemcpyAsync(bd, b, n * sizeof(double), hipMemcpyHostToDevice, ls->s));
-        PcgStats st = ls->pcg_na.solve(SysView{&ls->A, nullptr},
+        PcgStats st = ls->pcg_na.solve(SysView{&ls->A, nullptr, &ls->plan},
                                        ls->precond == SGIPC_PRECOND_MAS ? Precond::Mas
                                                                         : Precond::Diag,
                                        &ls->mas, bd, xd, pc, ls->s);

@@ -239,3 +239,74 @@ def test_mas_apply_workgroup_edges(oracle, nb, kind, prec):
     r = rng.normal(size=3 * nb)
     # FP32: inverses and sums of 48 products per level round at 6e-8 each
     assert rel(ls.precond(r), m.apply(r)) < (2e-5 if fp32 else 1e-10)
+
+
+def _spd_system(oracle, nb, seed, reach=40):
+    """A diagonally dominant block system with couplings to the next rows and
+    to random far ones (rows of 3 to about 20 blocks), 16-row parts."""
+    rng = np.random.default_rng(seed)
+    i = np.arange(nb)
+    pairs = [np.stack([i[:-d], i[d:]], 1) for d in (1, 3, 17, reach) if nb > d]
+    if nb > 4:
+        far = np.sort(rng.integers(0, nb, size=(2 * nb, 2)), axis=1)
+        pairs.append(far[far[:, 0] != far[:, 1]])
+    e = np.unique(np.concatenate(pairs), axis=0) if pairs else np.zeros((0, 2), np.int64)
+    off = 0.1 * rng.normal(size=(e.shape[0], 3, 3))
+    load = np.zeros(nb)
+    np.add.at(load, e.ravel(), np.abs(off).sum(axis=2).max(axis=1).repeat(2))
+    S = 0.1 * rng.normal(size=(nb, 3, 3))
+    diag = (1.2 * load + 0.5)[:, None, None] * np.eye(3) + S + S.transpose(0, 2, 1)
+    A = oracle.bsr_from_upper_triplets(nb, np.concatenate([i, e[:, 0]]),
+                                       np.concatenate([i, e[:, 1]]),
+                                       np.concatenate([diag, off]).reshape(-1, 9))
+    return A, (i // 16).astype(np.int32), rng.normal(size=3 * nb)
+
+
+@pytest.mark.parametrize("pc,prec", [("mas", "fp32"), ("mas", "fp64"), ("diag", "fp64")])
+@pytest.mark.parametrize("nb", [40, 63, 129, 700, 8200, 33000])
+def test_pcg_one_launch_sizes(oracle, nb, pc, prec):
+    """The one-launch solve at one workgroup, at the edges of its row ranges,
+    with one and two passes per row range and rows longer than it keeps in
+    registers: the solution of the system and the oracle's iterate after a
+    fixed number of iterations (max_iter is one more, as in the reference's
+    loop), with a stop test between."""
+    import sgipc
+    A, part, b = _spd_system(oracle, nb, nb)
+    ls = sgipc.LinearSystem(A.rowptr, A.cols, A.vals, part,
+                            sgipc.SGIPC_PRECOND_MAS if pc == "mas" else sgipc.SGIPC_PRECOND_DIAG,
+                            sgipc.SGIPC_MAS_FP32 if prec == "fp32" else sgipc.SGIPC_MAS_FP64)
+    for use_rz in (True, False):
+        x, st = ls.pcg(b, rel_tol=1e-12, use_rz=use_rz)
+        print(f"[one-launch] nb={nb} {pc} {prec} rz={use_rz} it={st.iterations} "
+              f"relres={st.rel_residual:.2e}", flush=True)
+        assert st.converged and st.iterations % 10 == 0
+        # the residual norm follows the tested norm up to the conditioning
+        # (about 10) of the preconditioned system
+        assert np.linalg.norm(A.spmv(x) - b) <= 1e-10 * np.linalg.norm(b)
+    if prec == "fp64":
+        m = oracle.Mas(A, part, fp32=False) if pc == "mas" else None
+        for cap in (1, 2, 8, 13):
+            x, st = ls.pcg(b, rel_tol=0.0, max_iter=cap)
+            xo, ito, _, _ = oracle.pcg(A, b, m, 1 if pc == "mas" else 0, rel_tol=0.0,
+                                       max_iter=cap)
+            assert st.iterations == ito == cap and not st.converged
+            # FP64 sums in another order, amplified by at most cap steps
+            assert np.linalg.norm(x - xo) <= 1e-11 * np.linalg.norm(xo)
+
+
+@pytest.mark.parametrize("pc", ["mas", "diag"])
+def test_pcg_beyond_one_launch(oracle, pc):
+    """More rows than the one-launch solve takes (256 per workgroup): a
+    launch per operation."""
+    import sgipc
+    A, part, b = _spd_system(oracle, 65700, 3)
+    ls = sgipc.LinearSystem(A.rowptr, A.cols, A.vals, part,
+                            sgipc.SGIPC_PRECOND_MAS if pc == "mas" else sgipc.SGIPC_PRECOND_DIAG,
+                            sgipc.SGIPC_MAS_FP64)
+    x, st = ls.pcg(b, rel_tol=1e-12)
+    assert st.converged
+    assert np.linalg.norm(A.spmv(x) - b) <= 1e-10 * np.linalg.norm(b)
+    m = oracle.Mas(A, part, fp32=False) if pc == "mas" else None
+    x, st = ls.pcg(b, rel_tol=0.0, max_iter=13)
+    xo, _, _, _ = oracle.pcg(A, b, m, 1 if pc == "mas" else 0, rel_tol=0.0, max_iter=13)
+    assert np.linalg.norm(x - xo) <= 1e-11 * np.linalg.norm(xo)
