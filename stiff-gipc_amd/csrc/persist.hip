@@ -241,7 +241,8 @@ __device__ __forceinline__ T mem_product(const T* __restrict__ S, int stride, co
 
 // LDS of a workgroup, in bytes, without the cached inverse rows and banks
 template <typename T>
-size_t persist_lds(int nloc, int nhalo, int nbank, const TailPlan& tp, int L, bool mas)
+size_t persist_lds(int nloc, int nhalo, int nbank, const TailPlan& tp, int L, bool mas,
+                   bool contact)
 {
     size_t n = (size_t)(6 * (nloc + nhalo) + 9 * nloc) * sizeof(double);
     if(mas)
@@ -252,6 +253,8 @@ size_t persist_lds(int nloc, int nhalo, int nbank, const TailPlan& tp, int L, bo
         n += (size_t)(nloc * ntl + nloc + 16 * nbank) * sizeof(short);
     }
     n += (size_t)nhalo * sizeof(int);
+    if(contact)
+        n += (size_t)3 * kPT * sizeof(double);
     return (n + 79) / 16 * 16;
 }
 
@@ -277,11 +280,12 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
     double*   rl  = xl + NV;
     double*   zl  = rl + NL3;
     double*   al  = zl + NL3;
+    double*   ce  = al + NL3;  // products of the contact blocks, one per thread
     const TailPlan& tp  = A.tp;
     const int       L   = A.L;
     const int       ntl = MAS ? L - tp.lt : 0;
     // tail R (kRB per bank), products of the tail nodes, r by level-0 slot
-    T*              Rs   = reinterpret_cast<T*>(al + NL3);
+    T*              Rs   = reinterpret_cast<T*>(ce + (A.rp2 ? 3 * kPT : 0));
     T*              zb   = Rs + kRB * (tp.span / BANK);
     T*              rs0  = zb + 3 * A.nloc * ntl;
     int*            hc   = reinterpret_cast<int*>(rs0 + (MAS ? kRB * A.nbank : 0));
@@ -400,56 +404,98 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
     }
     __syncthreads();
 
-    // al = A u for the own rows, u = [own | halo] in LDS; contact columns j
-    // through contact(j, c) from global memory; returns this thread's u.A u
+    // Contact rows are a few long ones (a body's nodes, a fixed vertex under a
+    // cloth): thread t takes the workgroup's t-th contact block, keeps its
+    // column's p in registers and leaves the product in ce for the row to
+    // sum in order; further blocks follow kPT at a time, their p read again.
+    int    e0 = 0, ne = 0, je = -1;
+    double pe[3] = {0.0, 0.0, 0.0};
+    if(A.rp2)
+    {
+        e0 = A.rp2[v0];
+        ne = A.rp2[v0 + nloc] - e0;
+        if(tid < ne)
+            je = A.cols2[e0 + tid];
+    }
+    auto contact_product = [&](int e, const double* u) {
+        const double* B = A.vals2 + 9 * (size_t)e;
+#pragma unroll
+        for(int c = 0; c < 3; c++)
+            ce[3 * tid + c] = B[3 * c] * u[0] + B[3 * c + 1] * u[1] + B[3 * c + 2] * u[2];
+    };
+
+    // al = A u for the own rows, u = [own | halo] in LDS, the first contact
+    // products in ce; contact columns j beyond them through contact(j, u_j)
+    // from global memory; returns this thread's u.A u
     auto spmv = [&](const double* u, auto&& contact) {
         const int g = tid % kRowL;
-        double    d = 0.0;
+        double    d = 0.0, a[kPasses][3];
+#pragma unroll
+        for(int s = 0; s < kPasses; s++)
+        {
+            a[s][0] = a[s][1] = a[s][2] = 0.0;
+            auto add = [&](const double* B, const double* x) {
+                const double x0 = x[0], x1 = x[1], x2 = x[2];
+                a[s][0] += B[0] * x0 + B[1] * x1 + B[2] * x2;
+                a[s][1] += B[3] * x0 + B[4] * x1 + B[5] * x2;
+                a[s][2] += B[6] * x0 + B[7] * x1 + B[8] * x2;
+            };
+#pragma unroll
+            for(int j = 0; j < kReg; j++)
+                add(Br[s][j], u + cr[s][j]);
+            for(int k = kn[s]; k < k1[s]; k += kRowL)
+            {
+                double B[9];
+#pragma unroll
+                for(int q = 0; q < 9; q++)
+                    B[q] = A.vals[9 * (size_t)k + q];
+                add(B, u + 3 * (int)A.lcol[k]);
+            }
+        }
+#pragma unroll 1
+        for(int h = 0; h < ne; h += kPT)
+        {
+            if(h > 0)
+            {
+                __syncthreads();
+                if(h + tid < ne)
+                {
+                    double x[3];
+                    contact(A.cols2[e0 + h + tid], x);
+                    contact_product(e0 + h + tid, x);
+                }
+                __syncthreads();
+            }
+#pragma unroll
+            for(int s = 0; s < kPasses; s++)
+                for(int k = q0[s] + (max(e0 + h - q0[s], 0) + kRowL - 1) / kRowL * kRowL;
+                    k < min(q1[s], e0 + h + kPT); k += kRowL)
+                {
+                    const double* c = ce + 3 * (k - e0 - h);
+                    a[s][0] += c[0];
+                    a[s][1] += c[1];
+                    a[s][2] += c[2];
+                }
+        }
 #pragma unroll
         for(int s = 0; s < kPasses; s++)
         {
             const int row = s * kPassRows + tid / kRowL;
-            double    a0 = 0, a1 = 0, a2 = 0;
-            auto      add = [&](const double* B, double x0, double x1, double x2) {
-                a0 += B[0] * x0 + B[1] * x1 + B[2] * x2;
-                a1 += B[3] * x0 + B[4] * x1 + B[5] * x2;
-                a2 += B[6] * x0 + B[7] * x1 + B[8] * x2;
-            };
-#pragma unroll
-            for(int j = 0; j < kReg; j++)
-                add(Br[s][j], u[cr[s][j]], u[cr[s][j] + 1], u[cr[s][j] + 2]);
-            for(int k = kn[s]; k < k1[s]; k += kRowL)
-            {
-                const double* x = u + 3 * (int)A.lcol[k];
-                double        B[9];
-#pragma unroll
-                for(int q = 0; q < 9; q++)
-                    B[q] = A.vals[9 * (size_t)k + q];
-                add(B, x[0], x[1], x[2]);
-            }
-            for(int k = q0[s]; k < q1[s]; k += kRowL)
-            {
-                double x0, x1, x2, B[9];
-                const int j = A.cols2[k];
-#pragma unroll
-                for(int q = 0; q < 9; q++)
-                    B[q] = A.vals2[9 * (size_t)k + q];
-                contact(j, x0, x1, x2);
-                add(B, x0, x1, x2);
-            }
 #pragma unroll
             for(int o = kRowL / 2; o > 0; o >>= 1)
             {
-                a0 += __shfl_xor(a0, o, kRowL);
-                a1 += __shfl_xor(a1, o, kRowL);
-                a2 += __shfl_xor(a2, o, kRowL);
+#pragma unroll
+                for(int c = 0; c < 3; c++)
+                    a[s][c] += __shfl_xor(a[s][c], o, kRowL);
             }
             if(row < nloc && g == 0)
             {
-                al[3 * row]     = a0;
-                al[3 * row + 1] = a1;
-                al[3 * row + 2] = a2;
-                d += u[3 * row] * a0 + u[3 * row + 1] * a1 + u[3 * row + 2] * a2;
+#pragma unroll
+                for(int c = 0; c < 3; c++)
+                {
+                    al[3 * row + c] = a[s][c];
+                    d += u[3 * row + c] * a[s][c];
+                }
             }
         }
         return d;
@@ -465,6 +511,13 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
             // ---- p = z + beta p: own rows and halo
             double* const       pnow = (k & 1) ? A.p1 : A.p0;
             const double* const pold = (k & 1) ? A.p0 : A.p1;
+            double ze[3] = {0.0, 0.0, 0.0};
+            if(je >= 0)
+            {
+#pragma unroll
+                for(int c = 0; c < 3; c++)
+                    ze[c] = ld_agent(A.z + 3 * (size_t)je + c);
+            }
             for(int i = tid; i < 3 * nh; i += kPT)
             {
                 const double zj = ld_agent(A.z + hc[i / 3] + i % 3);
@@ -477,17 +530,22 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
                 if(A.rp2)
                     st_agent(pnow + 3 * (size_t)v0 + i, p);
             }
+            if(je >= 0)
+            {
+#pragma unroll
+                for(int c = 0; c < 3; c++)
+                    pe[c] = fma(beta, pe[c], ze[c]);
+                contact_product(e0 + tid, pe);
+            }
             __syncthreads();
             // ---- A p and p.Ap
-            double pap = spmv(pl, [&](int j, double& x0, double& x1, double& x2) {
-                const double* zj = A.z + 3 * (size_t)j;
-                x0 = ld_agent(zj), x1 = ld_agent(zj + 1), x2 = ld_agent(zj + 2);
-                if(k > 1)
+            double pap = spmv(pl, [&](int j, double* p) {
+#pragma unroll
+                for(int c = 0; c < 3; c++)
                 {
-                    const double* pj = pold + 3 * (size_t)j;
-                    x0               = fma(beta, ld_agent(pj), x0);
-                    x1               = fma(beta, ld_agent(pj + 1), x1);
-                    x2               = fma(beta, ld_agent(pj + 2), x2);
+                    p[c] = ld_agent(A.z + 3 * (size_t)j + c);
+                    if(k > 1)
+                        p[c] = fma(beta, ld_agent(pold + 3 * (size_t)j + c), p[c]);
                 }
             });
             bar.arrive<1>(pap);
@@ -510,10 +568,19 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
                     break;
                 for(int i = tid; i < 3 * nh; i += kPT)
                     xl[n3 + i] = ld_agent(A.x + hc[i / 3] + i % 3);
+                if(je >= 0)
+                {
+                    double xe[3];
+#pragma unroll
+                    for(int c = 0; c < 3; c++)
+                        xe[c] = ld_agent(A.x + 3 * (size_t)je + c);
+                    contact_product(e0 + tid, xe);
+                }
                 __syncthreads();
-                spmv(xl, [&](int j, double& x0, double& x1, double& x2) {
-                    const double* xj = A.x + 3 * (size_t)j;
-                    x0 = ld_agent(xj), x1 = ld_agent(xj + 1), x2 = ld_agent(xj + 2);
+                spmv(xl, [&](int j, double* x) {
+#pragma unroll
+                    for(int c = 0; c < 3; c++)
+                        x[c] = ld_agent(A.x + 3 * (size_t)j + c);
                 });
                 __syncthreads();
                 for(int i = tid; i < n3; i += kPT)
@@ -642,17 +709,34 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
                     }
                     __syncthreads();
                 }
+                // four lanes per product
 #pragma unroll 1
-                for(int f = tid; f < 3 * total; f += kPT)
+                for(int f = tid / 4; f < 3 * total; f += kPT / 4)
                 {
-                    const int n  = list[f / 3];
-                    const T*  rv = Rs + kRB * (n / BANK);
+                    const int n  = list[f / 3], h = (BD / 4) * (tid % 4);
+                    const T*  rv = Rs + kRB * (n / BANK) + h;
+                    T         S[BD / 4], z = 0;
                     if(f < nkeep)
-                        zb[f] = lds_product(keep + kRow * f, 1, rv);
+                    {
+#pragma unroll
+                        for(int u = 0; u < BD / 4; u++)
+                            S[u] = keep[kRow * f + h + u];
+                    }
                     else
-                        zb[f] = mem_product(A.inv + (size_t)(b0 + n / BANK) * BD * BD
-                                                + (3 * (n % BANK) + f % 3) * BD,
-                                            1, rv);
+                    {
+                        const T* P = A.inv + (size_t)(b0 + n / BANK) * BD * BD
+                                     + (3 * (n % BANK) + f % 3) * BD + h;
+#pragma unroll
+                        for(int u = 0; u < BD / 4; u++)
+                            S[u] = P[u];
+                    }
+#pragma unroll
+                    for(int u = 0; u < BD / 4; u++)
+                        z += S[u] * rv[u];
+                    z += __shfl_xor(z, 1, 4);
+                    z += __shfl_xor(z, 2, 4);
+                    if(tid % 4 == 0)
+                        zb[f] = z;
                 }
                 __syncthreads();
             }
@@ -736,13 +820,14 @@ bool launch(PersistPlan& P, Mas* mas, PersistArgs<T> a, hipStream_t s)
         a.tp = tail_plan(a.L, mas->level_sizes(), [&](int span, int levels) {
             TailPlan t;
             t.lt = a.L - levels, t.span = span;
-            return persist_lds<T>(P.rows, P.halo, P.banks, t, a.L, true) <= kPLds;
+            return persist_lds<T>(P.rows, P.halo, P.banks, t, a.L, true, a.rp2 != nullptr)
+                   <= kPLds;
         });
         // the levels below the tail use the product buffer: 64 per wave
         if(a.tp.lt > 1 && 3 * P.rows * (a.L - a.tp.lt) < 64 * kPW)
             return false;
     }
-    const size_t fix = persist_lds<T>(P.rows, P.halo, P.banks, a.tp, a.L, MAS);
+    const size_t fix = persist_lds<T>(P.rows, P.halo, P.banks, a.tp, a.L, MAS, a.rp2 != nullptr);
     if(fix > kPLds)
         return false;
     a.keep_off     = (int)fix;
@@ -822,7 +907,7 @@ void PersistPlan::build(const Bsr& A, const std::vector<int>& part_first, hipStr
         hp[g + 1] = (int)hc.size();
         nh        = std::max(nh, hp[g + 1] - hp[g]);
     }
-    if(persist_lds<double>(nr, nh, nk, TailPlan{}, 0, false) > kPLds)
+    if(persist_lds<double>(nr, nh, nk, TailPlan{}, 0, false, true) > kPLds)
         return;
     rstart.upload(rs, s);
     bstart.upload(bs, s);

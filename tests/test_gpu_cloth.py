@@ -227,3 +227,29 @@ def test_cloth_over_affine_boxes_mixed_tracks_fp64(oracle):
             d0 = np.linalg.norm(x0[abd == b][:, None] - x0[abd == b][None], axis=2)
             d = np.linalg.norm(x[abd == b][:, None] - x[abd == b][None], axis=2)
             assert np.abs(d - d0).max() < 1e-6
+
+
+def test_newton_iteration_with_long_contact_rows(oracle):
+    """A sheet lying flat on the top face of a fixed box: the box's few
+    vertices carry the contact blocks of the whole sheet, more than a
+    workgroup of the one-launch solve takes in one round.  One Newton
+    iteration against the oracle (the scale of the iterates above)."""
+    import sgipc
+    from sgipc import scene as S
+    sc = S.cloth_scene(n=40, size=0.095, height=0.1013, n_boxes=1)
+    sc.mas_precision = sgipc.SGIPC_MAS_FP64
+    sim = sgipc.Simulation(sc)
+    w = oracle.World(sc)
+    sim.kappa = 1e4
+    w.kappa = 1e4
+    _, rowptr, cols, _ = sim.assemble()
+    box = np.setdiff1d(np.arange(sc.n_verts), sc.tris)
+    far = sum(int(np.isin(cols[rowptr[v]:rowptr[v + 1]], box, invert=True).sum()) for v in box)
+    st = sim.newton_iteration()
+    so = w.newton_iteration()
+    err = np.abs(sim.positions() - w.positions()).max() / np.abs(w.positions()).max()
+    print(f"[cloth-rows] box contact blocks={far} coo={sim.sizes()['coo_blocks']} "
+          f"pcg={st['pcg_iterations']}/{so['pcg_iterations']} err={err:.2e}", flush=True)
+    assert far > 512
+    assert abs(st["pcg_iterations"] - so["pcg_iterations"]) <= 10
+    assert err < 1e-6
