@@ -35,6 +35,22 @@ def test_mlp_loss_and_gradient_match_oracle(oracle):
     assert rel(g, go) < 1e-4
 
 
+@pytest.mark.parametrize("n", [1, 15, 63, 64, 65, 130])
+def test_mlp_gradient_batch_sizes(oracle, n):
+    """batches around the 64 samples that the weight gradient stages at a time"""
+    import sgipc
+    sim = sgipc.Simulation(_cubes())
+    rng = np.random.default_rng(n)
+    w = (rng.normal(size=NP) * 0.08).astype(np.float32)
+    X = rng.normal(size=(n, NI)).astype(np.float32)
+    T = rng.normal(size=(n, NO)).astype(np.float32)
+    sim.mlp_weights(w)
+    L, g = sim.mlp_loss_grad(X, T)
+    Lo, go = oracle.mlp_loss_grad(w, X, T)
+    assert L == pytest.approx(Lo, rel=1e-5)
+    assert rel(g, go) < 1e-4
+
+
 def test_mlp_training_reduces_loss(oracle):
     import sgipc
     sim = sgipc.Simulation(_cubes())
