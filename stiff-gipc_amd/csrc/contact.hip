@@ -9,16 +9,28 @@
 // (mlbvh.cu:537-1062, smooth == false).  Built with -ffp-contract=off so the
 // pair multiset equals the CPU restatement's.
 //
-// One wave per 64 queries; the traversal stack lives in LDS as stk[depth][lane]
-// (64 levels, the depth bound of a 64-bit-key Karras tree), so pushes and pops
-// are bank-conflict free.  Each record carries its raw candidate
-// (_ccd_collisionPair) for the CCD step bound.
+// One wave per 64 queries, one query per lane.  A traversal step loads one
+// 64-byte record (both children's boxes in FP32, rounded outwards); the exact
+// FP64 box test decides at the leaves, which gives the same leaves as FP64
+// tests all the way down (a leaf's box is inside its ancestors').  Proximity
+// and CCD queries skip subtrees whose primitives all belong to the query's
+// own body: such pairs are never candidates, and in scenes of many bodies
+// they are most of what a query meets.  Records are claimed with one counter
+// update per wave and event.  Bound by the dependent record loads: on 64 cubes
+// in contact (73,728 edges, 40,573 pairs) the edge-edge query takes 447 us
+// (646 us with separate node and box arrays in FP64, own-body subtrees
+// entered, and two counter updates per record).
+//
+// The traversal stack lives in LDS as stk[depth][lane] (bank-conflict free),
+// its rarely reached upper part (a 64-bit-key Karras tree is at most 64 deep)
+// in the lane's private memory.
 #include "sim_kernels.h"
 
 namespace sgipc
 {
 
-constexpr int kStack = 64;
+constexpr int kStackLds = 20;
+constexpr int kStackMax = 64;
 
 __device__ __forceinline__ bool overlap(const double* l, const double* r, double gap)
 {
@@ -29,6 +41,19 @@ __device__ __forceinline__ bool overlap(const double* l, const double* r, double
     return true;
 }
 
+// one counter update for the active lanes of the wave; this lane's slot
+__device__ __forceinline__ unsigned claim(unsigned* counter)
+{
+    const unsigned long long m      = __ballot(1);
+    const int                lane   = (int)__lane_id();
+    const int                leader = __ffsll((long long)m) - 1;
+    unsigned                 base   = 0;
+    if(lane == leader)
+        base = atomicAdd(counter, (unsigned)__popcll(m));
+    base = __shfl(base, leader, 64);
+    return base + (unsigned)__popcll(m & ((1ull << lane) - 1ull));
+}
+
 struct PairSink
 {
     int4*     pairs;
@@ -36,9 +61,10 @@ struct PairSink
     unsigned* cnt;  // [0] total, [2] PP, [3] PE, [4] PT + EE
     int       cap;
     int*      overflow;
+    unsigned  type[3] = {0, 0, 0};  // this lane's PP, PE, PT + EE records
     __device__ void emit(int4 code, int4 rawc, int slot_type)
     {
-        unsigned o = atomicAdd(cnt, 1u);
+        unsigned o = claim(cnt);
         if((int)o >= cap)
         {
             atomicExch(overflow, 1);
@@ -46,7 +72,21 @@ struct PairSink
         }
         pairs[o] = code;
         raw[o]   = rawc;
-        atomicAdd(cnt + slot_type, 1u);
+        type[0] += slot_type == 2 ? 1u : 0u;
+        type[1] += slot_type == 3 ? 1u : 0u;
+        type[2] += slot_type == 4 ? 1u : 0u;
+    }
+    // every lane of the wave, after its last record
+    __device__ void flush()
+    {
+        for(int k = 0; k < 3; k++)
+        {
+            unsigned t = type[k];
+            for(int o = 32; o > 0; o >>= 1)
+                t += __shfl_xor(t, o, 64);
+            if(__lane_id() == 0 && t)
+                atomicAdd(cnt + 2 + k, t);
+        }
     }
 };
 
@@ -182,71 +222,128 @@ __device__ __forceinline__ bool ee_ok(const int* body, const int* bt, uint2 a, u
     return true;
 }
 
-// generic stack traversal: visit(leaf_element) for every overlapping leaf.
-// With rng (each internal node's sorted leaf range) only leaves at sorted
-// positions above `after` are visited: a self query of the tree from its
-// sorted leaf `after` then meets every unordered pair of leaves once, from the
-// earlier one, and skips the subtrees that lie wholly at or before it.
+// what a traversal reads of a tree
+struct Tree
+{
+    int             n;
+    const NodeHalf* rec;
+    const double*   leaf;  // sorted leaf boxes
+    const uint64_t* keys;  // low word: element of the sorted leaf
+    __device__ uint32_t element(int s) const { return (uint32_t)keys[s]; }
+};
+
+static Tree tree_of(const Lbvh& b)
+{
+    return Tree{b.n, b.rec.data(), b.bvs.data() + 6 * (size_t)(b.n > 0 ? b.n - 1 : 0),
+                b.keys.data()};
+}
+
+// the float below / above x by at least one step
+__device__ __forceinline__ float below(double x)
+{
+    const float f = (float)x;
+    return f - fmaxf(fabsf(f) * 2.4e-7f, 1e-37f);
+}
+
+// visit(sorted leaf) for every leaf whose box overlaps q within gap, until it
+// returns true.  Leaves at sorted positions up to `after` are left out: a self
+// query of the tree from its sorted leaf `after` then meets every unordered
+// pair of leaves once, from the earlier one.  qbody: skip subtrees of this
+// body (kMixedBody: none).
 template <typename Visit>
-__device__ __forceinline__ void traverse(const uint32_t* __restrict__ nodes,
-                                         const double* __restrict__ bvs, int n, const double* q,
-                                         double gap, uint32_t (*stk)[64], Visit&& visit,
-                                         const int* __restrict__ rng = nullptr, int after = -1)
+__device__ __forceinline__ void traverse(const Tree& T, const double* q, double gap, int qbody,
+                                         uint32_t (*stk)[64], Visit&& visit, int after = -1)
 {
     const int lane = threadIdx.x;
-    if(n == 1)
+    if(after >= T.n - 1)
+        return;
+    if(T.n == 1)
     {
-        if(overlap(q, bvs, gap))
-            visit(nodes[3]);
+        if(overlap(q, T.leaf, gap))
+            visit(0);
         return;
     }
-    int sp          = 0;
-    stk[sp++][lane] = 0;
-    do
+    // the query box grown by gap and rounded outwards
+    float ql[3], qu[3];
+#pragma unroll
+    for(int c = 0; c < 3; c++)
     {
-        uint32_t node = stk[--sp][lane];
-        uint32_t ch[2] = {nodes[4 * (size_t)node + 1], nodes[4 * (size_t)node + 2]};
-        for(int c = 0; c < 2; c++)
+        qu[c] = -below(-(q[c] + gap));
+        ql[c] = below(q[3 + c] - gap);
+    }
+    auto hit = [&](const NodeHalf& h) {
+        bool ok = qbody == kMixedBody || h.body != qbody;
+#pragma unroll
+        for(int c = 0; c < 3; c++)
+            ok = ok && !(h.lo[c] > qu[c]) && !(h.up[c] < ql[c]);
+        return ok;
+    };
+    uint32_t deep[kStackMax - kStackLds];
+    int      sp   = 0;
+    uint32_t node = 0;
+    bool     more = true;
+    while(more)
+    {
+        const NodeHalf L = T.rec[2 * (size_t)node], R = T.rec[2 * (size_t)node + 1];
+        const bool     hl = hit(L) && (int)(L.child & 0x7fffffffu) > after, hr = hit(R);
+        const bool     ll = L.child >> 31, lr = R.child >> 31;
+        // the next node before the leaves' visits, which the lanes then
+        // reach together
+        const bool il = hl && !ll, ir = hr && !lr;
+        if(il && ir)
         {
-            uint32_t C = ch[c];
-            if(rng)
-            {
-                const int last = (int)C >= n - 1 ? (int)C - (n - 1) : rng[2 * (size_t)C + 1];
-                if(last <= after)
-                    continue;
-            }
-            if(!overlap(q, bvs + 6 * (size_t)C, gap))
-                continue;
-            uint32_t obj = nodes[4 * (size_t)C + 3];
-            if(obj != 0xFFFFFFFFu)
-                visit(obj);
-            else if(sp < kStack)
-                stk[sp++][lane] = C;
+            if(sp < kStackLds)
+                stk[sp++][lane] = R.child;
+            else if(sp < kStackMax)
+                deep[sp++ - kStackLds] = R.child;
         }
-    } while(sp > 0);
+        if(il || ir)
+            node = il ? L.child : R.child;
+        else if(sp == 0)
+            more = false;
+        else
+        {
+            sp--;
+            if(sp < kStackLds)
+                node = stk[sp][lane];
+            else
+                node = deep[sp - kStackLds];
+        }
+#pragma unroll 1
+        for(int h = 0; h < 2; h++)
+        {
+            const bool leaf = h == 0 ? hl && ll : hr && lr;
+            const int  s    = (int)((h == 0 ? L.child : R.child) & 0x7fffffffu);
+            if(leaf && overlap(q, T.leaf + 6 * (size_t)s, gap) && visit(s))
+                more = false;
+        }
+    }
 }
+
+__device__ __forceinline__ int query_body(int b) { return b == -1 ? kMixedBody : b; }
 
 __global__ void __launch_bounds__(64) k_query_vf(int ns, const uint32_t* __restrict__ surf,
                                                  const uint3* __restrict__ faces,
                                                  const int* __restrict__ body,
                                                  const int* __restrict__ bt,
-                                                 const double* __restrict__ x,
-                                                 const uint32_t* __restrict__ nodes,
-                                                 const double* __restrict__ bvs, int nf,
+                                                 const double* __restrict__ x, Tree tree,
                                                  double dHat, PairSink sk)
 {
-    __shared__ uint32_t stk[kStack][64];
+    __shared__ uint32_t stk[kStackLds][64];
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i >= ns)
-        return;
-    int    v    = (int)surf[i];
-    double q[6] = {x[3 * v], x[3 * v + 1], x[3 * v + 2], x[3 * v], x[3 * v + 1], x[3 * v + 2]};
-    double gap  = sqrt(dHat);
-    traverse(nodes, bvs, nf, q, gap, stk, [&](uint32_t obj) {
-        uint3 f = faces[obj];
-        if(vf_ok(body, bt, v, f))
-            check_pt(x, v, f.x, f.y, f.z, dHat, sk);
-    });
+    if(i < ns)
+    {
+        int    v    = (int)surf[i];
+        double q[6] = {x[3 * v], x[3 * v + 1], x[3 * v + 2], x[3 * v], x[3 * v + 1], x[3 * v + 2]};
+        double gap  = sqrt(dHat);
+        traverse(tree, q, gap, query_body(body[v]), stk, [&](int s) {
+            uint3 f = faces[tree.element(s)];
+            if(vf_ok(body, bt, v, f))
+                check_pt(x, v, f.x, f.y, f.z, dHat, sk);
+            return false;
+        });
+    }
+    sk.flush();
 }
 
 // Edge-edge pairs: each edge queries the edge tree from its own sorted leaf
@@ -256,34 +353,34 @@ __global__ void __launch_bounds__(64) k_query_ee(int ne, const uint2* __restrict
                                                  const int* __restrict__ body,
                                                  const int* __restrict__ bt,
                                                  const double* __restrict__ x,
-                                                 const double* __restrict__ xr,
-                                                 const uint32_t* __restrict__ nodes,
-                                                 const double* __restrict__ bvs,
-                                                 const int* __restrict__ rng, double dHat,
-                                                 PairSink sk)
+                                                 const double* __restrict__ xr, Tree tree,
+                                                 double dHat, PairSink sk)
 {
-    __shared__ uint32_t stk[kStack][64];
+    __shared__ uint32_t stk[kStackLds][64];
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i >= ne)
-        return;
-    int    leaf = i + ne - 1;
-    int    self = (int)nodes[4 * (size_t)leaf + 3];
-    double q[6];
-    for(int c = 0; c < 6; c++)
-        q[c] = bvs[6 * (size_t)leaf + c];
-    uint2  e   = edges[self];
-    double gap = sqrt(dHat);
-    traverse(
-        nodes, bvs, ne, q, gap, stk,
-        [&](uint32_t obj) {
-            const int lo = self < (int)obj ? self : (int)obj;
-            const int hi = self < (int)obj ? (int)obj : self;
-            uint2     o  = edges[obj];
-            uint2     a  = lo == self ? e : o, b = lo == self ? o : e;
-            if(ee_ok(body, bt, a, b, lo, hi))
-                check_ee(x, xr, a.x, a.y, b.x, b.y, hi, dHat, sk);
-        },
-        rng, i);
+    if(i < ne)
+    {
+        int    self = (int)tree.element(i);
+        double q[6];
+        for(int c = 0; c < 6; c++)
+            q[c] = tree.leaf[6 * (size_t)i + c];
+        uint2  e   = edges[self];
+        double gap = sqrt(dHat);
+        traverse(
+            tree, q, gap, query_body(body[e.x]), stk,
+            [&](int s) {
+                const int obj = (int)tree.element(s);
+                const int lo  = self < obj ? self : obj;
+                const int hi  = self < obj ? obj : self;
+                uint2     o   = edges[obj];
+                uint2     a = lo == self ? e : o, b = lo == self ? o : e;
+                if(ee_ok(body, bt, a, b, lo, hi))
+                    check_ee(x, xr, a.x, a.y, b.x, b.y, hi, dHat, sk);
+                return false;
+            },
+            i);
+    }
+    sk.flush();
 }
 
 struct CandSink
@@ -294,7 +391,7 @@ struct CandSink
     int*      overflow;
     __device__ void emit(int4 c)
     {
-        unsigned o = atomicAdd(cnt, 1u);
+        unsigned o = claim(cnt);
         if((int)o >= cap)
         {
             atomicExch(overflow, 1);
@@ -310,11 +407,9 @@ __global__ void __launch_bounds__(64) k_ccd_vf(int ns, const uint32_t* __restric
                                                const int* __restrict__ bt,
                                                const double* __restrict__ x,
                                                const double* __restrict__ dx, double alpha,
-                                               const uint32_t* __restrict__ nodes,
-                                               const double* __restrict__ bvs, int nf,
-                                               double dHat, CandSink sk)
+                                               Tree tree, double dHat, CandSink sk)
 {
-    __shared__ uint32_t stk[kStack][64];
+    __shared__ uint32_t stk[kStackLds][64];
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if(i >= ns)
         return;
@@ -327,45 +422,44 @@ __global__ void __launch_bounds__(64) k_ccd_vf(int ns, const uint32_t* __restric
         q[3 + c] = (b < a) ? b : a;
     }
     double gap = sqrt(dHat);
-    traverse(nodes, bvs, nf, q, gap, stk, [&](uint32_t obj) {
-        uint3 f = faces[obj];
+    traverse(tree, q, gap, query_body(body[v]), stk, [&](int s) {
+        uint3 f = faces[tree.element(s)];
         if(((body[v] != body[f.x]) || (body[v] == -1))
            && !(bt[v] >= 2 && bt[f.x] >= 2 && bt[f.y] >= 2 && bt[f.z] >= 2)
            && v != (int)f.x && v != (int)f.y && v != (int)f.z)
             sk.emit(make_int4(-v - 1, f.x, f.y, f.z));
+        return false;
     });
 }
 
 __global__ void __launch_bounds__(64) k_ccd_ee(int ne, const uint2* __restrict__ edges,
                                                const int* __restrict__ body,
-                                               const int* __restrict__ bt,
-                                               const uint32_t* __restrict__ nodes,
-                                               const double* __restrict__ bvs,
-                                               const int* __restrict__ rng, double dHat,
+                                               const int* __restrict__ bt, Tree tree, double dHat,
                                                CandSink sk)
 {
-    __shared__ uint32_t stk[kStack][64];
+    __shared__ uint32_t stk[kStackLds][64];
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if(i >= ne)
         return;
-    int    leaf = i + ne - 1;
-    int    self = (int)nodes[4 * (size_t)leaf + 3];
+    int    self = (int)tree.element(i);
     double q[6];
     for(int c = 0; c < 6; c++)
-        q[c] = bvs[6 * (size_t)leaf + c];
+        q[c] = tree.leaf[6 * (size_t)i + c];
     uint2  e   = edges[self];
     double gap = sqrt(dHat);
     traverse(
-        nodes, bvs, ne, q, gap, stk,
-        [&](uint32_t obj) {
-            const int lo = self < (int)obj ? self : (int)obj;
-            const int hi = self < (int)obj ? (int)obj : self;
-            uint2     o  = edges[obj];
-            uint2     a  = lo == self ? e : o, b = lo == self ? o : e;
+        tree, q, gap, query_body(body[e.x]), stk,
+        [&](int s) {
+            const int obj = (int)tree.element(s);
+            const int lo  = self < obj ? self : obj;
+            const int hi  = self < obj ? obj : self;
+            uint2     o   = edges[obj];
+            uint2     a = lo == self ? e : o, b = lo == self ? o : e;
             if(ee_ok(body, bt, a, b, lo, hi))
                 sk.emit(make_int4(a.x, a.y, b.x, b.y));
+            return false;
         },
-        rng, i);
+        i);
 }
 
 __device__ bool seg_tri(V3 e0, V3 e1, V3 t0, V3 t1, V3 t2)
@@ -388,39 +482,32 @@ __device__ bool seg_tri(V3 e0, V3 e1, V3 t0, V3 t1, V3 t2)
     return (u >= 0.0 && v >= 0.0 && u + v <= 1.0 && t >= 0.0 && t <= 1.0);
 }
 
+// one lane per face, in the face tree's sorted order (neighbouring lanes
+// walk neighbouring parts of the edge tree)
 __global__ void __launch_bounds__(64) k_edge_tri(int nf, const uint3* __restrict__ faces,
                                                  const uint2* __restrict__ edges,
                                                  const int* __restrict__ bt,
-                                                 const double* __restrict__ x,
-                                                 const uint32_t* __restrict__ nodes,
-                                                 const double* __restrict__ bvs, int ne, int* hit)
+                                                 const double* __restrict__ x, Tree ftree,
+                                                 Tree tree, int* hit)
 {
-    __shared__ uint32_t stk[kStack][64];
-    int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if(f >= nf)
+    __shared__ uint32_t stk[kStackLds][64];
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if(i >= nf)
         return;
-    uint3  F = faces[f];
-    double q[6] = {-1e32, -1e32, -1e32, 1e32, 1e32, 1e32};
-    uint32_t vs[3] = {F.x, F.y, F.z};
-    for(int k = 0; k < 3; k++)
-        for(int c = 0; c < 3; c++)
-        {
-            double p = x[3 * vs[k] + c];
-            q[3 + c] = (p < q[3 + c]) ? p : q[3 + c];
-            q[c]     = (q[c] < p) ? p : q[c];
-        }
+    uint3  F = faces[ftree.element(i)];
+    double q[6];
+    for(int c = 0; c < 6; c++)
+        q[c] = ftree.leaf[6 * (size_t)i + c];
     bool found = false;
-    traverse(nodes, bvs, ne, q, 0.0, stk, [&](uint32_t obj) {
-        if(found)
-            return;
-        uint2 E = edges[obj];
+    traverse(tree, q, 0.0, kMixedBody, stk, [&](int s) {
+        uint2 E = edges[tree.element(s)];
         if(F.x == E.x || F.x == E.y || F.y == E.x || F.y == E.y || F.z == E.x || F.z == E.y)
-            return;
+            return false;
         if(bt[F.x] >= 2 && bt[F.y] >= 2 && bt[F.z] >= 2 && bt[E.x] >= 2 && bt[E.y] >= 2)
-            return;
-        if(seg_tri(ld3(x + 3 * E.x), ld3(x + 3 * E.y), ld3(x + 3 * F.x), ld3(x + 3 * F.y),
-                   ld3(x + 3 * F.z)))
-            found = true;
+            return false;
+        found = seg_tri(ld3(x + 3 * E.x), ld3(x + 3 * E.y), ld3(x + 3 * F.x), ld3(x + 3 * F.y),
+                        ld3(x + 3 * F.z));
+        return found;
     });
     if(found)
         atomicExch(hit, 1);
@@ -446,12 +533,11 @@ void launch_query_proximity(const SimDev& d, const Lbvh& bf, const Lbvh& be, con
     PairSink sk{d.pairs, d.pairs_raw, d.pcount, d.pair_cap, d.overflow};
     if(d.nf > 0 && d.ns > 0)
         hipLaunchKernelGGL(k_query_vf, dim3(grid_for(d.ns, 64)), dim3(64), 0, s, d.ns, d.surf,
-                           (const uint3*)d.faces, d.body, d.btype, d.x, bf.nodes.data(),
-                           bf.bvs.data(), d.nf, d.dHat, sk);
+                           (const uint3*)d.faces, d.body, d.btype, d.x, tree_of(bf), d.dHat, sk);
     if(d.ne > 1)
         hipLaunchKernelGGL(k_query_ee, dim3(grid_for(d.ne, 64)), dim3(64), 0, s, d.ne,
-                           (const uint2*)d.edges, d.body, d.btype, d.x, xr, be.nodes.data(),
-                           be.bvs.data(), be.rng.data(), d.dHat, sk);
+                           (const uint2*)d.edges, d.body, d.btype, d.x, xr, tree_of(be), d.dHat,
+                           sk);
     SG_LAUNCH_CHECK();
 }
 
@@ -463,22 +549,21 @@ void launch_query_ccd(const SimDev& d, const Lbvh& bf, const Lbvh& be, const dou
     CandSink sk{cand, ccount, cap, overflow};
     if(d.nf > 0 && d.ns > 0)
         hipLaunchKernelGGL(k_ccd_vf, dim3(grid_for(d.ns, 64)), dim3(64), 0, s, d.ns, d.surf,
-                           (const uint3*)d.faces, d.body, d.btype, d.x, dx, alpha,
-                           bf.nodes.data(), bf.bvs.data(), d.nf, d.dHat, sk);
+                           (const uint3*)d.faces, d.body, d.btype, d.x, dx, alpha, tree_of(bf),
+                           d.dHat, sk);
     if(d.ne > 1)
         hipLaunchKernelGGL(k_ccd_ee, dim3(grid_for(d.ne, 64)), dim3(64), 0, s, d.ne,
-                           (const uint2*)d.edges, d.body, d.btype, be.nodes.data(), be.bvs.data(),
-                           be.rng.data(), d.dHat, sk);
+                           (const uint2*)d.edges, d.body, d.btype, tree_of(be), d.dHat, sk);
     SG_LAUNCH_CHECK();
 }
 
-void launch_edge_tri(const SimDev& d, const Lbvh& be, int* hit, hipStream_t s)
+void launch_edge_tri(const SimDev& d, const Lbvh& bf, const Lbvh& be, int* hit, hipStream_t s)
 {
     if(d.nf == 0 || d.ne == 0)
         return;
     hipLaunchKernelGGL(k_edge_tri, dim3(grid_for(d.nf, 64)), dim3(64), 0, s, d.nf,
-                       (const uint3*)d.faces, (const uint2*)d.edges, d.btype, d.x,
-                       be.nodes.data(), be.bvs.data(), d.ne, hit);
+                       (const uint3*)d.faces, (const uint2*)d.edges, d.btype, d.x, tree_of(bf),
+                       tree_of(be), hit);
     SG_LAUNCH_CHECK();
 }
 

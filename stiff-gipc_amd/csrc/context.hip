@@ -747,8 +747,8 @@ Context::Context(const sgipc_scene_desc& d)
     // (ABDPreconditioner on the body range after the global 3x3 diagonal)
     if(nabd_ > 0)
         pcg_.set_bodies(nfem_, nabd_, bslots_.data());
-    bf_.init(nf_, 3, faces_.data());
-    be_.init(ne_, 2, edges_.data());
+    bf_.init(nf_, 3, faces_.data(), body_.data());
+    be_.init(ne_, 2, edges_.data(), body_.data());
     build_bvh();
     build_cp();
     SG_HIP(hipStreamSynchronize(s_));
@@ -982,7 +982,7 @@ bool Context::is_intersected()
     SG_HIP(hipStreamSynchronize(s_));
     if(h)
         return true;
-    launch_edge_tri(dev_, be_, hit, s_);
+    launch_edge_tri(dev_, bf_, be_, hit, s_);
     SG_HIP(hipMemcpyAsync(&h, hit, sizeof(int), hipMemcpyDeviceToHost, s_));
     SG_HIP(hipStreamSynchronize(s_));
     return h != 0;

@@ -13,6 +13,9 @@
 // lane the mask of same-digit peers, per-wave digit counts are combined in
 // LDS.  Digits above the index width and above the 30-bit Morton code are
 // skipped, so a 50k-primitive tree needs 6 passes.
+#include <climits>
+
+#include "sgipc.h"
 #include "sim_kernels.h"
 
 namespace sgipc
@@ -280,8 +283,9 @@ __global__ void __launch_bounds__(kSortThreads) k_sort_scatter(int n, int shift,
 __device__ __forceinline__ int cub64(uint64_t a, uint64_t b) { return __clzll(a ^ b); }
 
 __global__ void k_leaf_nodes(int n, const uint64_t* __restrict__ keys, uint32_t* __restrict__ nodes,
-                             const double* __restrict__ leaf, double* __restrict__ bvs,
-                             unsigned* __restrict__ flags)
+                             const double* __restrict__ leaf, double* __restrict__ bvs, int arity,
+                             const uint32_t* __restrict__ prims, const int* __restrict__ body,
+                             int2* __restrict__ lbody)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if(i >= n)
@@ -290,12 +294,13 @@ __global__ void k_leaf_nodes(int n, const uint64_t* __restrict__ keys, uint32_t*
     {
         uint32_t* nd = nodes + 4 * (size_t)i;
         nd[0] = nd[1] = nd[2] = nd[3] = 0xFFFFFFFFu;
-        flags[i]                      = 0u;
     }
     uint32_t  el = (uint32_t)(keys[i] & 0xFFFFFFFFull);
     uint32_t* nd = nodes + 4 * (size_t)(i + n - 1);
     nd[0] = nd[1] = nd[2] = 0xFFFFFFFFu;
     nd[3]                 = el;
+    const int b = body[prims[(size_t)arity * el]];
+    lbody[i]    = make_int2(b, b);
     for(int c = 0; c < 6; c++)
         bvs[6 * (size_t)(i + n - 1) + c] = leaf[6 * (size_t)el + c];
 }
@@ -384,45 +389,28 @@ __global__ void k_internal_nodes(int n, const uint64_t* __restrict__ code, uint3
 // box is the union of those leaf boxes.  Unions are exact (max/min), so the
 // boxes are bit-identical to a bottom-up refit whatever the order.  Instead
 // of walking up with atomics and device-wide fences, every node is computed
-// independently from leaf boxes and two levels of precomputed aggregates:
-// blocks of 64 leaves and super-blocks of 64 blocks.
-constexpr int kAgg = 64;
+// independently from the aligned power-of-two groups of leaves (level k: one
+// box per 2^k leaves): a range is at most two groups per level, so the longest
+// chain is 2 log2(n) boxes.  (With two levels of 64-groups a node scanned up
+// to 255 boxes one after the other: 84 us per tree of 387k edges.)  The
+// groups also carry the smallest and largest body id of their primitives.
 
-struct Box6
+// one thread per entry of the input level (m entries); a wave makes the six
+// levels above it
+__global__ void __launch_bounds__(256) k_box_levels(int m, const double* __restrict__ in,
+                                                    const int2* __restrict__ inb,
+                                                    double* __restrict__ agg,
+                                                    int2* __restrict__ aggb, BoxLevels lv, int k0)
 {
-    double u[3], l[3];
-};
-
-__device__ __forceinline__ Box6 box_empty()
-{
-    Box6 b;
-    for(int c = 0; c < 3; c++)
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    double    v[6];
+    int2      b = make_int2(INT_MAX, INT_MIN);
+    if(i < m)
     {
-        b.u[c] = -INFINITY;
-        b.l[c] = INFINITY;
-    }
-    return b;
-}
-
-__device__ __forceinline__ void box_add(Box6& b, const double* p)  // p: {upper, lower}
-{
-    for(int c = 0; c < 3; c++)
-    {
-        double a = p[c], d = p[3 + c];
-        b.u[c]   = (b.u[c] < a) ? a : b.u[c];
-        b.l[c]   = (d < b.l[c]) ? d : b.l[c];
-    }
-}
-
-// one wave per group of 64 input boxes: out[g] = union of in[64 g .. 64 g + 63]
-__global__ void __launch_bounds__(256) k_box_groups(int n, const double* __restrict__ in,
-                                                    double* __restrict__ out)
-{
-    int    i = blockIdx.x * blockDim.x + threadIdx.x;
-    double v[6];
-    if(i < n)
         for(int c = 0; c < 6; c++)
             v[c] = in[6 * (size_t)i + c];
+        b = inb[i];
+    }
     else
         for(int c = 0; c < 3; c++)
         {
@@ -430,7 +418,9 @@ __global__ void __launch_bounds__(256) k_box_groups(int n, const double* __restr
             v[3 + c] = INFINITY;
         }
 #pragma unroll
-    for(int o = 32; o > 0; o >>= 1)
+    for(int k = 0; k < 6; k++)
+    {
+        const int o = 1 << k;
 #pragma unroll
         for(int c = 0; c < 3; c++)
         {
@@ -438,71 +428,127 @@ __global__ void __launch_bounds__(256) k_box_groups(int n, const double* __restr
             v[c]     = (v[c] < a) ? a : v[c];
             v[3 + c] = (d < v[3 + c]) ? d : v[3 + c];
         }
-    int g = i >> 6;
-    if((i & 63) < 6 && g < (n + 63) / 64)
-        out[6 * (size_t)g + (i & 63)] = v[i & 63];
-}
-
-// union of in[a .. b] (inclusive)
-__device__ __forceinline__ void box_scan(Box6& acc, const double* __restrict__ in, int a, int b)
-{
-    for(int j = a; j <= b; j++)
-        box_add(acc, in + 6 * (size_t)j);
-}
-
-__global__ void __launch_bounds__(256) k_refit_query(int n, const int* __restrict__ rng,
-                                                     const double* __restrict__ blk,
-                                                     const double* __restrict__ sup,
-                                                     double* __restrict__ bvs)
-{
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i >= n - 1)
-        return;
-    const double* leaf = bvs + 6 * (size_t)(n - 1);
-    int           f = rng[2 * (size_t)i], l = rng[2 * (size_t)i + 1];
-    Box6          acc = box_empty();
-    if(l - f < 2 * kAgg)
-        box_scan(acc, leaf, f, l);
-    else
-    {
-        int fb = (f + kAgg - 1) / kAgg, lb = (l + 1) / kAgg - 1;  // full blocks fb..lb
-        box_scan(acc, leaf, f, fb * kAgg - 1);
-        box_scan(acc, leaf, (lb + 1) * kAgg, l);
-        if(lb - fb < 2 * kAgg)
-            box_scan(acc, blk, fb, lb);
-        else
+        b.x = min(b.x, __shfl_xor(b.x, o, 64));
+        b.y = max(b.y, __shfl_xor(b.y, o, 64));
+        if(i < m && (i & (2 * o - 1)) == 0)
         {
-            int fs = (fb + kAgg - 1) / kAgg, ls = (lb + 1) / kAgg - 1;  // full super-blocks
-            box_scan(acc, blk, fb, fs * kAgg - 1);
-            box_scan(acc, blk, (ls + 1) * kAgg, lb);
-            box_scan(acc, sup, fs, ls);
+            const size_t g = (size_t)lv.off[k0 + k + 1] + (i >> (k + 1));
+#pragma unroll
+            for(int c = 0; c < 6; c++)
+                agg[6 * g + c] = v[c];
+            aggb[g] = b;
         }
     }
-    double* o = bvs + 6 * (size_t)i;
-    for(int c = 0; c < 3; c++)
-    {
-        o[c]     = acc.u[c];
-        o[3 + c] = acc.l[c];
-    }
 }
 
-void Lbvh::init(int n_, int arity_, const uint32_t* prims_)
+// the next float below / above x unless x is a float
+__device__ __forceinline__ float float_down(double x)
+{
+    float f = (float)x;
+    if((double)f > x)
+        f = f > 0.0f ? __uint_as_float(__float_as_uint(f) - 1u)
+                     : (f < 0.0f ? __uint_as_float(__float_as_uint(f) + 1u) : -1e-45f);
+    return f;
+}
+__device__ __forceinline__ float float_up(double x) { return -float_down(-x); }
+
+// one thread per node: internal nodes' boxes, and every node's half of its
+// parent's traversal record (box rounded outwards to FP32)
+__global__ void __launch_bounds__(256) k_refit(int n, const int* __restrict__ rng,
+                                               const uint32_t* __restrict__ nodes,
+                                               const int2* __restrict__ lbody,
+                                               const double* __restrict__ agg,
+                                               const int2* __restrict__ aggb, BoxLevels lv,
+                                               double* __restrict__ bvs,
+                                               NodeHalf* __restrict__ rec)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if(i >= 2 * n - 1)
+        return;
+    const uint32_t parent = nodes[4 * (size_t)i];
+    const double*  leaf   = bvs + 6 * (size_t)(n - 1);
+    double         v[6];
+    int2           b;
+    if(i >= n - 1)
+    {
+        for(int c = 0; c < 6; c++)
+            v[c] = bvs[6 * (size_t)i + c];
+        b = lbody[i - (n - 1)];
+    }
+    else
+    {
+        for(int c = 0; c < 3; c++)
+        {
+            v[c]     = -INFINITY;
+            v[3 + c] = INFINITY;
+        }
+        b        = make_int2(INT_MAX, INT_MIN);
+        auto add = [&](int k, int j) {
+            const double* p = k == 0 ? leaf + 6 * (size_t)j : agg + 6 * (size_t)(lv.off[k] + j);
+            const int2    q = k == 0 ? lbody[j] : aggb[lv.off[k] + j];
+#pragma unroll
+            for(int c = 0; c < 3; c++)
+            {
+                v[c]     = (v[c] < p[c]) ? p[c] : v[c];
+                v[3 + c] = (p[3 + c] < v[3 + c]) ? p[3 + c] : v[3 + c];
+            }
+            b.x = min(b.x, q.x);
+            b.y = max(b.y, q.y);
+        };
+        int l = rng[2 * (size_t)i], r = rng[2 * (size_t)i + 1] + 1;
+        for(int k = 0; l < r; k++)
+        {
+            if(l & 1)
+                add(k, l++);
+            if(r & 1)
+                add(k, --r);
+            l >>= 1;
+            r >>= 1;
+        }
+        double* o = bvs + 6 * (size_t)i;
+        for(int c = 0; c < 6; c++)
+            o[c] = v[c];
+    }
+    if(parent == 0xFFFFFFFFu)
+        return;
+    NodeHalf h;
+    for(int c = 0; c < 3; c++)
+    {
+        h.up[c] = float_up(v[c]);
+        h.lo[c] = float_down(v[3 + c]);
+    }
+    h.child = i >= n - 1 ? (0x80000000u | (uint32_t)(i - (n - 1))) : (uint32_t)i;
+    h.body  = b.x == b.y && b.x != -1 ? b.x : kMixedBody;
+    rec[2 * (size_t)parent + (nodes[4 * (size_t)parent + 1] == (uint32_t)i ? 0 : 1)] = h;
+}
+
+void Lbvh::init(int n_, int arity_, const uint32_t* prims_, const int* body_)
 {
     n     = n_;
     arity = arity_;
     prims = prims_;
+    body  = body_;
     if(n <= 0)
         return;
     leaf.resize(6 * (size_t)n);
     bvs.resize(6 * (size_t)(2 * n - 1));
     nodes.resize(4 * (size_t)(2 * n - 1));
+    rec.resize(2 * (size_t)(n > 1 ? n - 1 : 1));
     keys.resize(n);
     keys_alt.resize(n);
-    flags.resize(n);
+    lbody.resize(n);
     rng.resize(2 * (size_t)(n > 1 ? n - 1 : 1));
-    int nblk_agg = (n + kAgg - 1) / kAgg;
-    agg_blk.resize(6 * (size_t)nblk_agg);
-    agg_sup.resize(6 * (size_t)((nblk_agg + kAgg - 1) / kAgg));
+    levels    = BoxLevels{};
+    int total = 0, m = n;
+    // six levels per launch, past the first level of one box
+    for(int k = 1; k < kBoxLevels; k++)
+    {
+        m             = (m + 1) / 2;
+        levels.off[k] = total;
+        total += m;
+    }
+    agg.resize(6 * (size_t)total);
+    aggb.resize(total);
     hist.resize(radix_sort_hist_size(n));
     scene.resize(6);
     partial.resize(6 * (size_t)grid_for(n, 256));
@@ -602,18 +648,25 @@ void Lbvh::build(const double* x, const double* dx, double alpha, hipStream_t s)
     // 30 Morton bits alone orders by (morton, index)
     radix_sort_keys(keys.data(), keys_alt.data(), hist.data(), n, 32, 62, s);
     hipLaunchKernelGGL(k_leaf_nodes, dim3(grid_for(n, 256)), dim3(256), 0, s, n, keys.data(),
-                       nodes.data(), leaf.data(), bvs.data(), flags.data());
+                       nodes.data(), leaf.data(), bvs.data(), arity, prims, body, lbody.data());
     if(n > 1)
     {
         hipLaunchKernelGGL(k_internal_nodes, dim3(grid_for(n - 1, 256)), dim3(256), 0, s, n,
                            keys.data(), nodes.data(), rng.data());
-        int nblk_agg = (n + kAgg - 1) / kAgg;
-        hipLaunchKernelGGL(k_box_groups, dim3(grid_for(n, 256)), dim3(256), 0, s, n,
-                           bvs.data() + 6 * (size_t)(n - 1), agg_blk.data());
-        hipLaunchKernelGGL(k_box_groups, dim3(grid_for(nblk_agg, 256)), dim3(256), 0, s,
-                           nblk_agg, agg_blk.data(), agg_sup.data());
-        hipLaunchKernelGGL(k_refit_query, dim3(grid_for(n - 1, 256)), dim3(256), 0, s, n,
-                           rng.data(), agg_blk.data(), agg_sup.data(), bvs.data());
+        int m = n;
+        for(int k = 0; m > 1; k += 6)
+        {
+            SG_CHECK(k + 6 < kBoxLevels, SGIPC_ECAPACITY, "too many primitives for the box levels");
+            hipLaunchKernelGGL(k_box_levels, dim3(grid_for(m, 256)), dim3(256), 0, s, m,
+                               k == 0 ? bvs.data() + 6 * (size_t)(n - 1)
+                                      : agg.data() + 6 * (size_t)levels.off[k],
+                               k == 0 ? lbody.data() : aggb.data() + levels.off[k], agg.data(),
+                               aggb.data(), levels, k);
+            m = (m + 63) / 64;
+        }
+        hipLaunchKernelGGL(k_refit, dim3(grid_for(2 * n - 1, 256)), dim3(256), 0, s, n, rng.data(),
+                           nodes.data(), lbody.data(), agg.data(), aggb.data(), levels, bvs.data(),
+                           rec.data());
     }
     SG_LAUNCH_CHECK();
 }

@@ -184,21 +184,43 @@ size_t scan_tmp_size(int n);
 void spatial_sort_keys(int kind, const double* x, int nv, const uint32_t* tets, int nt,
                        uint64_t* keys_out, uint32_t* order_out, hipStream_t s);
 
+// Traversal record of an internal node: its two children, 32 bytes each, so a
+// step of a traversal is one 64-byte load.  The FP32 box contains the child's
+// FP64 box.  child: node id, or 0x80000000 | sorted leaf; of a left child it is
+// (Karras) also the last sorted leaf below it.  body: the body id of every
+// primitive below, kMixedBody when they differ (or have none, -1).
+constexpr int kMixedBody = -0x7fffffff - 1;
+struct alignas(32) NodeHalf
+{
+    float    lo[3], up[3];
+    uint32_t child;
+    int      body;
+};
+// offsets of the levels of aligned leaf groups (level k: 2^k leaves per box)
+constexpr int kBoxLevels = 31;
+struct BoxLevels
+{
+    int off[kBoxLevels];
+};
+
 // lbvh.hip: linear BVH over faces (arity 3) or edges (arity 2)
 struct Lbvh
 {
     int               n = 0, arity = 0;
     const uint32_t*   prims = nullptr;
+    const int*        body  = nullptr;  // body id per vertex
     DBuf<double>      leaf;    // 6 n
     DBuf<double>      bvs;     // 6 (2n - 1) {upper, lower}
     DBuf<uint32_t>    nodes;   // 4 (2n - 1) {parent, left, right, element}
     DBuf<uint64_t>    keys, keys_alt;
-    DBuf<unsigned>    flags;
-    DBuf<int>         rng;                // 2 (n - 1): sorted leaf range of each internal node
-    DBuf<double>      agg_blk, agg_sup;   // unions of 64 leaves / of 64 such blocks
+    DBuf<NodeHalf>    rec;     // 2 (n - 1)
+    DBuf<int>         rng;     // 2 (n - 1): sorted leaf range of each internal node
+    DBuf<double>      agg;     // boxes of the leaf groups, level by level
+    DBuf<int2>        aggb, lbody;  // smallest and largest body of the groups / leaves
+    BoxLevels         levels;
     DBuf<unsigned>    hist;
     DBuf<double>      scene, partial;
-    void init(int n, int arity, const uint32_t* prims);
+    void init(int n, int arity, const uint32_t* prims, const int* body);
     // swept boxes when dx != nullptr: box(x) U box(x - alpha dx)
     void build(const double* x, const double* dx, double alpha, hipStream_t s);
 };
@@ -211,7 +233,7 @@ void launch_query_proximity(const SimDev& d, const Lbvh& bf, const Lbvh& be, con
 void launch_query_ccd(const SimDev& d, const Lbvh& bf, const Lbvh& be, const double* dx,
                       double alpha, int4* cand, unsigned* ccount, int cap, int* overflow,
                       hipStream_t s);
-void launch_edge_tri(const SimDev& d, const Lbvh& be, int* hit, hipStream_t s);
+void launch_edge_tri(const SimDev& d, const Lbvh& bf, const Lbvh& be, int* hit, hipStream_t s);
 void launch_ground_intersect(const SimDev& d, int* hit, hipStream_t s);
 
 // ccd.hip: reductions write max(1/toc) style values into out (positive max)

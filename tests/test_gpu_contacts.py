@@ -130,3 +130,45 @@ def test_ccd_bound_impact(oracle):
         co = w.ccd_candidates(dx, a)
         print(f"[impact] candidates alpha={a:.4g}: {len(cg)}", flush=True)
         assert len(cg) > 0 and _key(cg) == _key(co)
+
+
+@pytest.mark.parametrize("n", [2, 3, 6, 9, 12, 33])
+@pytest.mark.parametrize("which", [0, 1])
+def test_lbvh_tree_sizes(oracle, n, which):
+    """trees of 2 to about 3,100 primitives, around the multiples of 64 leaves
+    of the refit's groups: keys, nodes and boxes bit for bit"""
+    import sgipc
+    from sgipc import scene as S
+    sc = S.cloth_scene(n=n, size=0.02 * n, n_boxes=0)
+    x = sc.x + 1e-3 * np.random.default_rng(n).normal(size=sc.x.shape)
+    sim = sgipc.Simulation(sc)
+    sim.set_positions(x)
+    k, nd, bv = sim.lbvh(which)
+    ko, ndo, bvo = oracle.lbvh(x, sc.faces if which == 0 else sc.edges)
+    print(f"[lbvh-size] n={ko.size}", flush=True)
+    np.testing.assert_array_equal(k, ko)
+    np.testing.assert_array_equal(nd, ndo)
+    np.testing.assert_array_equal(bv.view(np.uint64), bvo.view(np.uint64))
+
+
+@pytest.mark.parametrize("ids", ["distinct", "same", "none", "mixed"])
+def test_contacts_by_body_id(oracle, ids):
+    """four cubes within a large contact distance, their vertices of distinct
+    bodies, of one body (no pairs), of none (self contact of every cube), or
+    of one body, none, and two others: the pairs of the brute-force search"""
+    import sgipc
+    from sgipc import scene as S
+    sc = S.stack_scene(n=4, cells=2, size=0.1, gap=0.01, dhat=0.02)
+    of = {"distinct": (0, 1, 2, 3), "same": (5, 5, 5, 5), "none": (-1, -1, -1, -1),
+          "mixed": (7, -1, 7, 3)}[ids]
+    sc.body_id = np.asarray(of, np.int32)[sc.body_id]
+    x = sc.x + 1e-4 * np.random.default_rng(0).normal(size=sc.x.shape)
+    sim = sgipc.Simulation(sc)
+    sim.set_positions(x)
+    pairs, counts, _ = sim.contacts()
+    pb, cb = oracle.contact_pairs(sc, x, "brute")
+    key = lambda p: sorted(map(tuple, np.asarray(p).tolist()))
+    print(f"[contact-bodies] {ids} pairs={counts.tolist()}", flush=True)
+    assert (counts[0] > 0) == (ids != "same")
+    assert key(pairs) == key(pb)
+    np.testing.assert_array_equal(counts, cb)
