@@ -134,8 +134,11 @@ inline bool mas_blocked_invert()
     return e && strcmp(e, "blocked") == 0;
 }
 
-void launch_mas_invert_gj(const double* B, float* inv, int nbanks, hipStream_t s);
-void launch_mas_invert_gj(const double* B, double* inv, int nbanks, hipStream_t s);
+// packed inverses of all banks, dense ones of the banks from first_dense
+void launch_mas_invert_gj(const double* B, float* inv, float* dense, int first_dense, int nbanks,
+                          hipStream_t s);
+void launch_mas_invert_gj(const double* B, double* inv, double* dense, int first_dense,
+                          int nbanks, hipStream_t s);
 
 // the bank matrices of MAS levels >= 1 from the Galerkin operators A_l,
 // summed in a fixed order by sorting (mas_galerkin.hip)
@@ -164,7 +167,7 @@ struct MasView
 {
     const int *     vert_of_slot, *going_next, *bank_first, *bank_ncl, *chain, *child_bank;
     const unsigned* child_mask;
-    const T*        inv;
+    const T *       inv, *dense;  // packed; coarse banks dense
     T *             R, *Z;
 };
 
@@ -202,6 +205,7 @@ class Mas
     template <typename T>
     MasView<T> view();
     bool       fp32() const { return cfg_.fp32; }
+    int        parts() const { return nparts_; }  // level-0 banks
     // first row of each part (size parts + 1)
     const std::vector<int>& part_first() const { return part_first_; }
     int levels() const { return L_; }
@@ -223,7 +227,7 @@ class Mas
                        const double* pap, V* z, double* rz_out, double* zero0, double* zero1,
                        const int* done, hipStream_t s, bool defer_rz);
     template <typename T, typename V>
-    void apply_levels(const T* inv, T* R, T* Z, V* x, V* r, const V* p, const V* Ap,
+    void apply_levels(const T* inv, const T* dense, T* R, T* Z, V* x, V* r, const V* p, const V* Ap,
                       const double* rz_prev, const double* pap, V* z, double* rz_out,
                       double* zero0, double* zero1, const int* done, hipStream_t s,
                       bool defer_rz);
@@ -247,8 +251,8 @@ class Mas
     DBuf<int>      lvl_;       // 2 * (L + 1): count, offset
     std::vector<int> h_lvl_;
     DBuf<double>   B_;         // nbanks x 48 x 48 assembled (FP64)
-    DBuf<float>    inv32_;
-    DBuf<double>   inv64_;
+    DBuf<float>    inv32_, dense32_;  // packed inverses; the coarse banks' dense ones
+    DBuf<double>   inv64_, dense64_;
     DBuf<float>    R32_, Z32_;
     DBuf<double>   R64_, Z64_;
     DBuf<int>      going_next_; // global id -> global id one level up

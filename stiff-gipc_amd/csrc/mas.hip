@@ -371,7 +371,8 @@ __device__ __forceinline__ void tile_store(double* S, int r0, int c0, dbl4 t)
 }
 
 template <typename T>
-__global__ void __launch_bounds__(64) k_mas_invert(const double* __restrict__ B, T* __restrict__ inv)
+__global__ void __launch_bounds__(64) k_mas_invert(const double* __restrict__ B, T* __restrict__ inv,
+                                                   T* __restrict__ dense, int first_dense)
 {
     __shared__ double S[BD * kInvLd];
     const int     bank = blockIdx.x;
@@ -455,38 +456,24 @@ __global__ void __launch_bounds__(64) k_mas_invert(const double* __restrict__ B,
             wave_lds_sync();
         }
     }
-    // Stored transposed (dst[u][t] = Binv[t][u], so that the lanes of a wave
-    // read a row with unit stride), keeping only the upper 3x3 blocks of the
-    // inverse, as the reference's MasMatrixSymf does (eigen_data.h:125-128,
-    // written by __inverse6_P96x96, MASPreconditioner.cu:628-724): below the
-    // block diagonal the operator is the transpose of the upper blocks
-    T* dst = inv + (size_t)bank * BD * BD;
-    for(int e = l; e < BD * BD; e += 64)
+    // the symmetric matrix of the upper triangle (the reference keeps the
+    // upper 3x3 blocks of the inverse, MasMatrixSymf, eigen_data.h:125-128,
+    // written by __inverse6_P96x96, MASPreconditioner.cu:628-724)
+    auto at = [&](int r, int c) {
+        return (T)S[(r < c ? r : c) * kInvLd + (r < c ? c : r)];
+    };
+    T* dst = inv + (size_t)bank * kBankPack;
+    for(int e = l; e < kBankPack; e += 64)
+        dst[e] = at(e % BD, (e % BD + e / BD) % BD);
+    if(bank >= first_dense)
     {
-        int r = e / BD, c = e % BD;
-        dst[e] = (T)((r / 3 >= c / 3) ? S[c * kInvLd + r] : S[r * kInvLd + c]);
+        T* dd = dense + (size_t)(bank - first_dense) * BD * BD;
+        for(int e = l; e < BD * BD; e += 64)
+            dd[e] = at(e / BD, e % BD);
     }
 }
 
 // ---------------------------------------------------------------- apply
-template <typename T>
-__device__ __forceinline__ T bank_apply(const T (&pv)[BD], T rv)
-{
-    T acc = 0;
-#pragma unroll
-    for(int u = 0; u < BD; u++)
-        acc += pv[u] * __shfl(rv, u, 64);
-    return acc;
-}
-
-template <typename T>
-__device__ __forceinline__ T bank_product(const T* __restrict__ inv, int gb, T rv)
-{
-    T pv[BD];
-    bank_load(inv, gb, pv);
-    return bank_apply(pv, rv);
-}
-
 // Cluster sums of one bank's R into the next level, stored (the bank owns
 // those nodes).  rv: lane t < 48 holds component t % 3 of bank node t / 3;
 // node_up: global id of that node's parent (or -1).  Lane t < 3 ncl sums
@@ -563,8 +550,8 @@ __global__ void __launch_bounds__(64) k_mas_l0(const int* __restrict__ vert_of_s
         ncl   = bank_ncl[b];
     }
     const int gn = *((has_coarse && t < BD) ? going_next + s : bank_ncl + b);
-    T         pv[BD];
-    bank_load(inv, b, pv);
+    BankRow<T> pv;
+    pv.load(inv, b);
     double a = 0.0;
     if(x)
         a = wave_sum(ra) / wave_sum(pa);  // slot_set_sum of both sets
@@ -582,16 +569,13 @@ __global__ void __launch_bounds__(64) k_mas_l0(const int* __restrict__ vert_of_s
             rv -= av * Ap[d];
         }
     }
-    // z = Binv r with r broadcast from LDS (12 ds_read_b128 instead of 48
-    // cross-lane permutes; same products, same order)
-    __shared__ T Rs[64];
-    T rt  = (T)rv;
-    Rs[t] = rt;
+    // z = Binv r with r in LDS
+    __shared__ T Rs[2 * BD];
+    T rt = (T)rv;
+    if(t < BD)
+        Rs[t] = Rs[t + BD] = rt;
     wave_lds_sync();
-    T z = 0;
-#pragma unroll
-    for(int u = 0; u < BD; u++)
-        z += pv[u] * Rs[u];
+    const T z = pv.product(Rs);
     Z[(size_t)b * ZB + t] = z;
     if(x && v >= 0)
     {
@@ -622,7 +606,13 @@ __global__ void __launch_bounds__(64) k_mas_lx(int bank0, int node0, int count,
     const int cc    = t % 3;
     const bool valid = (t < BD) && (g - node0 < count);
     T         rv    = valid ? R[3 * (size_t)g + cc] : (T)0;
-    T         z     = bank_product(inv, gb, rv);
+    BankRow<T> pv;
+    pv.load(inv, gb);
+    __shared__ T Rs[2 * BD];
+    if(t < BD)
+        Rs[t] = Rs[t + BD] = rv;
+    wave_lds_sync();
+    const T z = pv.product(Rs);
     Z[(size_t)gb * ZB + t] = z;
     if(has_next)
         restrict_bank(Rc, rv, valid ? going_next[g] : -1, bank_first[gb], bank_ncl[gb], R);
@@ -660,8 +650,8 @@ template <typename T, typename V, int NL>
 __global__ void __launch_bounds__(kFinThreads)
     k_mas_finish(int nv, TailPlan tp, const int* __restrict__ slot_of,
                  const int* __restrict__ chain, const int* __restrict__ child_bank,
-                 const unsigned* __restrict__ child_mask, const T* __restrict__ inv,
-                 const T* __restrict__ R, const T* __restrict__ Z, const V* __restrict__ r,
+                 const unsigned* __restrict__ child_mask, const T* __restrict__ dense,
+                 int first_dense, const T* __restrict__ R, const T* __restrict__ Z, const V* __restrict__ r,
                  V* __restrict__ z, double* rz_out, double* zero0, double* zero1,
                  const int* __restrict__ done)
 {
@@ -776,7 +766,7 @@ __global__ void __launch_bounds__(kFinThreads)
         if(tid < 3 * total)
         {
             const int n = list[tid / 3];
-            row_load(inv, b0 + n / BANK, 3 * (n % BANK) + tid % 3, pv);
+            row_load(dense, b0 - first_dense + n / BANK, 3 * (n % BANK) + tid % 3, pv);
         }
     }
     if(stop)
@@ -817,7 +807,7 @@ __global__ void __launch_bounds__(kFinThreads)
         {
             const int n = list[f / 3];
             if(f >= kFinThreads)
-                row_load(inv, b0 + n / BANK, 3 * (n % BANK) + f % 3, pv);
+                row_load(dense, b0 - first_dense + n / BANK, 3 * (n % BANK) + f % 3, pv);
             zb[f] = row_product(pv, Rs + 3 * BANK * (n / BANK));
         }
         __syncthreads();
@@ -994,13 +984,15 @@ void Mas::build(const SysView& S, hipStream_t s)
         B_.resize(nbanks * BD * BD);
         if(cfg_.fp32)
         {
-            inv32_.resize(nbanks * BD * BD);
+            inv32_.resize(nbanks * kBankPack);
+            dense32_.resize((nbanks - nparts_) * BD * BD);
             R32_.resize(3 * (size_t)total_clusters_);
             Z32_.resize((size_t)ZB * nbanks);
         }
         else
         {
-            inv64_.resize(nbanks * BD * BD);
+            inv64_.resize(nbanks * kBankPack);
+            dense64_.resize((nbanks - nparts_) * BD * BD);
             R64_.resize(3 * (size_t)total_clusters_);
             Z64_.resize((size_t)ZB * nbanks);
         }
@@ -1040,19 +1032,28 @@ void Mas::bank_host(int bank, double* mat, double* inv, hipStream_t s) const
     if(mat)
         SG_HIP(hipMemcpyAsync(mat, B_.data() + off, 48 * 48 * sizeof(double),
                               hipMemcpyDeviceToHost, s));
-    if(inv && !cfg_.fp32)
-        SG_HIP(hipMemcpyAsync(inv, inv64_.data() + off, 48 * 48 * sizeof(double),
-                              hipMemcpyDeviceToHost, s));
-    std::vector<float> f;
+    std::vector<float>  f;
+    std::vector<double> g;
+    const size_t        po = (size_t)bank * kBankPack;
     if(inv && cfg_.fp32)
     {
-        f.resize(48 * 48);
-        SG_HIP(hipMemcpyAsync(f.data(), inv32_.data() + off, 48 * 48 * sizeof(float),
+        f.resize(kBankPack);
+        SG_HIP(hipMemcpyAsync(f.data(), inv32_.data() + po, kBankPack * sizeof(float),
+                              hipMemcpyDeviceToHost, s));
+    }
+    else if(inv)
+    {
+        g.resize(kBankPack);
+        SG_HIP(hipMemcpyAsync(g.data(), inv64_.data() + po, kBankPack * sizeof(double),
                               hipMemcpyDeviceToHost, s));
     }
     SG_HIP(hipStreamSynchronize(s));
-    for(size_t i = 0; i < f.size(); i++)
-        inv[i] = f[i];
+    if(inv)
+        for(int i = 0; i < BD * BD; i++)
+        {
+            const int k = pack_at(i / BD, i % BD);
+            inv[i]      = cfg_.fp32 ? (double)f[k] : g[k];
+        }
 }
 
 void Mas::invert(hipStream_t s)
@@ -1064,16 +1065,18 @@ void Mas::invert(hipStream_t s)
     {
         // scalar Gauss-Jordan in the reference's order (mas_invert.hip)
         if(cfg_.fp32)
-            launch_mas_invert_gj(B_.data(), inv32_.data(), (int)nbanks, s);
+            launch_mas_invert_gj(B_.data(), inv32_.data(), dense32_.data(), nparts_,
+                                 (int)nbanks, s);
         else
-            launch_mas_invert_gj(B_.data(), inv64_.data(), (int)nbanks, s);
+            launch_mas_invert_gj(B_.data(), inv64_.data(), dense64_.data(), nparts_,
+                                 (int)nbanks, s);
     }
     else if(cfg_.fp32)
         hipLaunchKernelGGL(k_mas_invert<float>, dim3(nbanks), dim3(64), 0, s, B_.data(),
-                           inv32_.data());
+                           inv32_.data(), dense32_.data(), nparts_);
     else
         hipLaunchKernelGGL(k_mas_invert<double>, dim3(nbanks), dim3(64), 0, s, B_.data(),
-                           inv64_.data());
+                           inv64_.data(), dense64_.data(), nparts_);
     if(prof)
         prof->end("mas_invert", s);
     SG_LAUNCH_CHECK();
@@ -1085,7 +1088,7 @@ void Mas::invert(hipStream_t s)
 // iteration with the tail at level 2, 45.0 at level 4; 173,225 rows: 104.4 at
 // level 2, 107.9 at level 3).
 template <typename T, typename V>
-void Mas::apply_levels(const T* inv, T* R, T* Z, V* x, V* r, const V* p, const V* Ap,
+void Mas::apply_levels(const T* inv, const T* dense, T* R, T* Z, V* x, V* r, const V* p, const V* Ap,
                        const double* rz_prev, const double* pap, V* z, double* rz_out,
                        double* zero0, double* zero1, const int* done, hipStream_t s,
                        bool defer_rz)
@@ -1114,7 +1117,7 @@ void Mas::apply_levels(const T* inv, T* R, T* Z, V* x, V* r, const V* p, const V
         hipLaunchKernelGGL(kern, dim3(grid_for(nv_, kFinThreads)), dim3(kFinThreads),
                            tp.lt < L_ ? finish_lds<T>(tp.span, L_ - tp.lt) : 64, s, nv_, tp,
                            slot_of_.data(), chain_.data(), child_bank_.data(),
-                           child_mask_.data(), inv, R, Z, r, z, rz_out, zero0, zero1, done);
+                           child_mask_.data(), dense, nparts_, R, Z, r, z, rz_out, zero0, zero1, done);
     };
     static_assert(kMaxLevels == 6, "the dispatch below covers 1 .. 6 levels");
     switch(L_)
@@ -1138,10 +1141,10 @@ void Mas::apply_fused_t(V* x, V* r, const V* p, const V* Ap, const double* rz_pr
 {
     SG_CHECK(built_, -5, "MAS apply before build");
     if(cfg_.fp32)
-        apply_levels<float, V>(inv32_.data(), R32_.data(), Z32_.data(), x, r, p, Ap, rz_prev, pap,
+        apply_levels<float, V>(inv32_.data(), dense32_.data(), R32_.data(), Z32_.data(), x, r, p, Ap, rz_prev, pap,
                                z, rz_out, zero0, zero1, done, s, defer_rz);
     else
-        apply_levels<double, V>(inv64_.data(), R64_.data(), Z64_.data(), x, r, p, Ap, rz_prev,
+        apply_levels<double, V>(inv64_.data(), dense64_.data(), R64_.data(), Z64_.data(), x, r, p, Ap, rz_prev,
                                 pap, z, rz_out, zero0, zero1, done, s, defer_rz);
 }
 
@@ -1171,14 +1174,14 @@ template <>
 MasView<float> Mas::view<float>()
 {
     return {vert_of_slot_.data(), going_next_.data(), bank_first_.data(), bank_ncl_.data(),
-            chain_.data(), child_bank_.data(), child_mask_.data(), inv32_.data(), R32_.data(),
+            chain_.data(), child_bank_.data(), child_mask_.data(), inv32_.data(), dense32_.data(), R32_.data(),
             Z32_.data()};
 }
 template <>
 MasView<double> Mas::view<double>()
 {
     return {vert_of_slot_.data(), going_next_.data(), bank_first_.data(), bank_ncl_.data(),
-            chain_.data(), child_bank_.data(), child_mask_.data(), inv64_.data(), R64_.data(),
+            chain_.data(), child_bank_.data(), child_mask_.data(), inv64_.data(), dense64_.data(), R64_.data(),
             Z64_.data()};
 }
 

@@ -20,11 +20,12 @@
 // so every register index is static and nothing goes to scratch.
 //
 // Output: the symmetric matrix built from the inverse's upper triangle,
-// out[r][c] = Binv[min(r, c)][max(r, c)].  The reference keeps the upper 3x3
+// out[r][c] = Binv[min(r, c)][max(r, c)], packed by diagonals (mas_tail.h) and,
+// for the coarse banks, dense as well.  The reference keeps the upper 3x3
 // blocks (MasMatrixSymf, eigen_data.h:125-128) after copying each diagonal
 // block's upper entries below its diagonal (MASPreconditioner.cu:704-708); the
 // operator it applies is exactly this matrix.
-#include "linsys.h"
+#include "mas_tail.h"
 
 namespace sgipc
 {
@@ -106,7 +107,8 @@ struct GjStep<kBD>
 
 template <typename T>
 __global__ void __launch_bounds__(64) k_mas_invert_gj(const double* __restrict__ B,
-                                                     T* __restrict__ inv)
+                                                     T* __restrict__ inv, T* __restrict__ dense,
+                                                     int first_dense)
 {
     __shared__ GjShared sh;
     __shared__ double   S[kBD * kLd];
@@ -135,29 +137,41 @@ __global__ void __launch_bounds__(64) k_mas_invert_gj(const double* __restrict__
             S[(kTR * g + r) * kLd + kTC * h + c] = a[r][c];
     }
     __syncthreads();
-    T* dst = inv + (size_t)bank * kBD * kBD;
-    for(int e = lane; e < kBD * kBD; e += 64)
+    auto at = [&](int r, int q) {
+        return (T)S[(r < q ? r : q) * kLd + (r < q ? q : r)];
+    };
+    T* dst = inv + (size_t)bank * kBankPack;
+    for(int e = lane; e < kBankPack; e += 64)
     {
-        const int r = e / kBD, q = e % kBD;
-        const int lo = r < q ? r : q, hi = r < q ? q : r;
-        dst[e]       = (T)S[lo * kLd + hi];
+        const int d = e / kBD, t = e % kBD;
+        dst[e]      = at(t, (t + d) % kBD);
+    }
+    if(bank >= first_dense)
+    {
+        T* dd = dense + (size_t)(bank - first_dense) * kBD * kBD;
+        for(int e = lane; e < kBD * kBD; e += 64)
+            dd[e] = at(e / kBD, e % kBD);
     }
 }
 }  // namespace
 
-void launch_mas_invert_gj(const double* B, float* inv, int nbanks, hipStream_t s)
+void launch_mas_invert_gj(const double* B, float* inv, float* dense, int first_dense, int nbanks,
+                          hipStream_t s)
 {
     if(nbanks < 1)
         return;
-    hipLaunchKernelGGL(k_mas_invert_gj<float>, dim3(nbanks), dim3(64), 0, s, B, inv);
+    hipLaunchKernelGGL(k_mas_invert_gj<float>, dim3(nbanks), dim3(64), 0, s, B, inv, dense,
+                       first_dense);
     SG_LAUNCH_CHECK();
 }
 
-void launch_mas_invert_gj(const double* B, double* inv, int nbanks, hipStream_t s)
+void launch_mas_invert_gj(const double* B, double* inv, double* dense, int first_dense, int nbanks,
+                          hipStream_t s)
 {
     if(nbanks < 1)
         return;
-    hipLaunchKernelGGL(k_mas_invert_gj<double>, dim3(nbanks), dim3(64), 0, s, B, inv);
+    hipLaunchKernelGGL(k_mas_invert_gj<double>, dim3(nbanks), dim3(64), 0, s, B, inv, dense,
+                       first_dense);
     SG_LAUNCH_CHECK();
 }
 

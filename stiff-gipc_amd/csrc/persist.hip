@@ -55,6 +55,11 @@ constexpr int kMaxGroups = 256;
 // iteration takes 13.1 / 13.6 / 17.1 us on 425 rows, 15.1 / 13.5 / 19.6 us on
 // 6,480 rows (FP64 MAS), 9.6 / 8.5 / 10.3 us on 7,560 rows (block Jacobi)
 constexpr int kGroupRows = 64;
+// Rows that a level-0 bank counts for when the rows are shared out: the waves
+// take one bank product each at a time, and banks hold 3 .. 16 rows.  By rows
+// alone the workgroups of a 43,264-row system get up to 25 banks, 17 on
+// average, and wait for the largest; with 8 rows per bank up to 22
+constexpr int kBankRows  = 8;
 constexpr int kSlotWords = 4;              // two doubles in four words
 constexpr int kMaxPolls  = 1 << 22;
 // R of a 16-node bank in LDS takes 50 entries instead of 48: the members of
@@ -62,6 +67,7 @@ constexpr int kMaxPolls  = 1 << 22;
 // on the same LDS banks
 constexpr int kRB  = 50;
 constexpr int kRow = BD + 1;  // cached inverse row
+constexpr int kR0  = 2 * BD + 2;  // r of a level-0 bank, twice in a row
 constexpr size_t kPLds   = 156 * 1024;     // LDS of a workgroup at most
 
 template <typename T>
@@ -92,9 +98,9 @@ struct PersistArgs
     // MAS
     const int *     vert_of_slot, *bank_first, *bank_ncl, *chain, *child_bank;
     const unsigned* child_mask;
-    const T*        inv;
+    const T *       inv, *dense;
     T *             R, *Z;
-    int             L, nbank;
+    int             L, nbank, first_dense;
     TailPlan        tp;
     // stop test
     double rel2, abs2, q_ref;
@@ -207,35 +213,48 @@ struct Barrier
     }
 };
 
-// sum_u S[u * stride] rv[u] over a bank's 48 entries, S and rv in LDS
+// z_t of a packed bank inverse S (LDS or global memory) for lane t < 48 (lanes
+// above: a copy of lane 0's), R: the bank's values twice in a row in LDS.
+// In parts of 96 bytes, so that the values fit beside the matrix blocks
+// in the registers.
 template <typename T>
-__device__ __forceinline__ T lds_product(const T* S, int stride, const T* rv)
+__device__ __forceinline__ T packed_product(const T* __restrict__ S, const T* R)
 {
-    T z = 0;
-#pragma unroll 12
-    for(int u = 0; u < BD; u++)
-        z += S[u * stride] * rv[u];
+    const int l = (int)__lane_id(), t = l < BD ? l : 0;
+    T         z = S[t] * R[t];
+    constexpr int N = 48 / sizeof(T);
+#pragma unroll 1
+    for(int h = 1; h < kDiag; h += N)
+    {
+        T a[N], m[N];
+#pragma unroll
+        for(int k = 0; k < N; k++)
+        {
+            const int d = h + k;
+            a[k]        = S[(unsigned)(d * BD + t)];
+            m[k]        = S[(unsigned)(d * BD + (t >= d ? t - d : t - d + BD))];
+        }
+#pragma unroll
+        for(int k = 0; k < N; k++)
+        {
+            z += a[k] * R[t + h + k];
+            if(h + k < kDiag - 1)  // D_24 holds both its halves
+                z += m[k] * R[t - h - k + BD];
+        }
+    }
     return z;
 }
 
-// the same with S in global memory, loaded in parts that fit beside the
-// matrix blocks in the registers
+// the same with S whole, in LDS: fewer LDS reads, for r is the same for all
+// lanes (425 rows, an iteration: 13.8 us packed, 13.3 us whole)
 template <typename T>
-__device__ __forceinline__ T mem_product(const T* __restrict__ S, int stride, const T* rv)
+__device__ __forceinline__ T whole_product(const T* S, const T* R)
 {
-    T             z = 0;
-    constexpr int N = 96 / sizeof(T);
-#pragma unroll
-    for(int h = 0; h < BD; h += N)
-    {
-        T pv[N];
-#pragma unroll
-        for(int u = 0; u < N; u++)
-            pv[u] = S[(h + u) * stride];
-#pragma unroll
-        for(int u = 0; u < N; u++)
-            z += pv[u] * rv[h + u];
-    }
+    S += __lane_id() < BD ? __lane_id() : 0;
+    T z = 0;
+#pragma unroll 12
+    for(int u = 0; u < BD; u++)
+        z += S[u * BD] * R[u];
     return z;
 }
 
@@ -248,7 +267,8 @@ size_t persist_lds(int nloc, int nhalo, int nbank, const TailPlan& tp, int L, bo
     if(mas)
     {
         const int ntl = L - tp.lt;
-        n += (size_t)(kRB * (tp.span / BANK) + 3 * nloc * ntl + kRB * nbank) * sizeof(T);
+        n += (size_t)(kRB * (tp.span / BANK) + std::max(3 * nloc * ntl, 2 * BD * kPW) + kR0 * nbank)
+             * sizeof(T);
         n += (size_t)(nloc * ntl + (tp.span - tp.first) + nloc) * sizeof(int);
         n += (size_t)(nloc * ntl + nloc + 16 * nbank) * sizeof(short);
     }
@@ -287,8 +307,8 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
     // tail R (kRB per bank), products of the tail nodes, r by level-0 slot
     T*              Rs   = reinterpret_cast<T*>(ce + (A.rp2 ? 3 * kPT : 0));
     T*              zb   = Rs + kRB * (tp.span / BANK);
-    T*              rs0  = zb + 3 * A.nloc * ntl;
-    int*            hc   = reinterpret_cast<int*>(rs0 + (MAS ? kRB * A.nbank : 0));
+    T*              rs0  = zb + (MAS ? max(3 * A.nloc * ntl, 2 * BD * kPW) : 0);
+    int*            hc   = reinterpret_cast<int*>(rs0 + (MAS ? kR0 * A.nbank : 0));
     int*            list = hc + A.nhalo;
     unsigned*       memb = reinterpret_cast<unsigned*>(list + A.nloc * ntl);
     unsigned*       own1 = memb + (tp.span - tp.first);
@@ -306,7 +326,10 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
     }
     for(int i = tid; i < nh; i += kPT)
         hc[i] = 3 * A.hcol[h0 + i];
-    int nkeep = 0, nbcache = 0;  // cached rows of tail products, cached level-0 banks
+    int  nkeep = 0, nbcache = 0;  // cached rows of tail products, cached level-0 banks
+    bool whole  = false;          // the latter as 48 x 48 blocks
+    int  nstage = 0;              // banks loaded again each iteration, into stage
+    T*   stage  = nullptr;
     if constexpr(MAS)
     {
         bk0 = A.bstart[b], nbk = A.bstart[b + 1] - bk0;
@@ -315,9 +338,9 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
             const int v = A.vert_of_slot[16 * (size_t)bk0 + i];
             lsl[i]      = v >= 0 ? (unsigned short)(v - v0) : (unsigned short)0xffff;
             if(v >= 0)
-                at0[v - v0] = (unsigned short)(kRB * (i / BANK) + 3 * (i % BANK));
+                at0[v - v0] = (unsigned short)(kR0 * (i / BANK) + 3 * (i % BANK));
         }
-        for(int i = tid; i < kRB * A.nbank; i += kPT)
+        for(int i = tid; i < kR0 * A.nbank; i += kPT)
             rs0[i] = (T)0;
         // own level-1 nodes (consecutive): member slots
         if(nbk > 0)
@@ -359,19 +382,48 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
         for(int f = tid / 16; f < nkeep; f += kPT / 16)
         {
             const int n = list[f / 3];
-            const T*  P = A.inv + (size_t)(b0 + n / BANK) * BD * BD + (3 * (n % BANK) + f % 3) * BD;
+            const T*  P = A.dense + (size_t)(b0 - A.first_dense + n / BANK) * BD * BD
+                         + (3 * (n % BANK) + f % 3) * BD;
             for(int u = tid % 16; u < BD; u += 16)
                 keep[kRow * f + u] = P[u];
         }
-        nbcache = min(nbk, (A.cache - kRow * nkeep) / (BD * BD));
-        for(int i = tid; i < nbcache * BD * BD; i += kPT)
-            keep[kRow * nkeep + i] = A.inv[(size_t)bk0 * BD * BD + i];
+        const int left = A.cache - kRow * nkeep;
+        whole          = nbk * BD * BD <= left;
+        nbcache        = whole ? nbk : min(nbk, left / kBankPack);
+        for(int i = tid; i < nbcache * (whole ? BD * BD : kBankPack); i += kPT)
+            keep[kRow * nkeep + i] =
+                whole ? A.inv[(size_t)(bk0 + i / (BD * BD)) * kBankPack
+                              + pack_at(i % (BD * BD) / BD, i % BD)]
+                      : A.inv[(size_t)bk0 * kBankPack + i];
+        stage  = reinterpret_cast<T*>(((size_t)Rs + 15) & ~(size_t)15);
+        nstage = min(nbk - nbcache, (int)(rs0 - stage) / kBankPack);
     }
+    // The inverses that found no place for the whole solve come into the
+    // tail's buffers, which are free until level 0 is done, while the
+    // workgroup waits at a barrier. 1 KB per wave and step; a step that would
+    // end beyond the last bank starts earlier.  43,264 rows, an iteration: 24.6
+    // us with these banks read where they are used, 21.4 us (with kBankRows).
+    auto load_stage = [&]() {
+        if constexpr(MAS)
+        {
+            constexpr int V = 16 / sizeof(T);  // values per lane
+            const T*      p = A.inv + (size_t)(bk0 + nbcache) * kBankPack;
+            const int     n = nstage * kBankPack;
+            for(int i = 64 * V * w; i < n; i += 64 * V * kPW)
+            {
+                const int o = min(i, n - 64 * V);
+                __builtin_amdgcn_global_load_lds(
+                    (const __attribute__((address_space(1))) void*)(p + o + V * lane),
+                    (__attribute__((address_space(3))) void*)(stage + o), 16, 0, 0);
+            }
+        }
+    };
     __syncthreads();
+    load_stage();
     auto put_r = [&](int i, double r) {
         rl[i] = r;
         if constexpr(MAS)
-            rs0[at0[i / 3] + i % 3] = (T)r;
+            rs0[at0[i / 3] + i % 3] = rs0[at0[i / 3] + i % 3 + BD] = (T)r;
     };
     for(int i = tid; i < n3; i += kPT)
         put_r(i, A.b[3 * (size_t)v0 + i]);
@@ -549,6 +601,7 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
                 }
             });
             bar.arrive<1>(pap);
+            load_stage();
             if(!bar.wait<1>(&pap))
                 break;
             // ---- x += a p, r -= a Ap; at a check r = b - A x
@@ -586,8 +639,9 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
                 for(int i = tid; i < n3; i += kPT)
                     put_r(i, A.b[3 * (size_t)v0 + i] - al[i]);
             }
-            __syncthreads();
         }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the staged inverses
+        __syncthreads();
         if(!A.use_rz && (check || k == 0))
             for(int i = tid; i < n3; i += kPT)
                 rr += rl[i] * rl[i];
@@ -616,7 +670,7 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
             for(int q = tid; q < 3 * n1; q += kPT)
             {
                 const unsigned mk = own1[q / 3];
-                const T        s  = member_sum(rs0 + kRB * (mk >> 16), mk, q % 3);
+                const T        s  = member_sum(rs0 + kR0 * (mk >> 16), mk, q % 3);
                 st_agent(A.R + 3 * (size_t)f0 + q, s);
             }
             bar.arrive<0>();
@@ -624,13 +678,16 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
 #pragma unroll 1
             for(int j = w; j < nbk; j += kPW)
             {
-                const T* rv = rs0 + kRB * j;
-                const T  z  = j < nbcache
-                                  ? lds_product(keep + kRow * nkeep + j * BD * BD + (lane < BD ? lane : 0),
-                                                BD, rv)
-                                  : mem_product(A.inv + (size_t)(bk0 + j) * BD * BD
-                                                    + (lane < BD ? lane : 0),
-                                                BD, rv);
+                const T* rv = rs0 + kR0 * j;
+                T        z;
+                if(whole)
+                    z = whole_product(keep + kRow * nkeep + j * BD * BD, rv);
+                else if(j < nbcache + nstage)
+                    z = packed_product(j < nbcache ? keep + kRow * nkeep + j * kBankPack
+                                                   : stage + (j - nbcache) * kBankPack,
+                                       rv);
+                else
+                    z = packed_product(A.inv + (size_t)(bk0 + j) * kBankPack, rv);
                 const int sl = lane < BD ? (int)lsl[16 * j + lane / 3] : 0xffff;
                 if(sl != 0xffff)
                     zl[3 * sl + lane % 3] = (double)z;
@@ -648,13 +705,14 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
                     const int  gb    = tp.off[l] / BANK + j;
                     const int  g     = gb * BANK + lane / 3;
                     const bool valid = lane < BD && g - tp.off[l] < tp.count[l];
-                    T*         Rv    = zb + 64 * w;  // free until the tail's products
+                    T*         Rv    = zb + 2 * BD * w;  // free until the tail's products
                     wave_lds_sync();
-                    Rv[lane] = valid ? ld_agent(A.R + 3 * (size_t)g + lane % 3) : (T)0;
+                    if(lane < BD)
+                        Rv[lane] = Rv[lane + BD] =
+                            valid ? ld_agent(A.R + 3 * (size_t)g + lane % 3) : (T)0;
                     wave_lds_sync();
                     st_agent(A.Z + (size_t)gb * ZB + lane,
-                             mem_product(A.inv + (size_t)gb * BD * BD + (lane < BD ? lane : 0),
-                                         BD, Rv));
+                             packed_product(A.inv + (size_t)gb * kBankPack, Rv));
                     if(l + 1 < L)
                     {
                         const int first = A.bank_first[gb], ncl = A.bank_ncl[gb];
@@ -701,10 +759,13 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
                 {
                     const int o = tp.off[l + 1] - tp.base;
 #pragma unroll 1
-                    for(int q = tid; q < 3 * tp.count[l + 1]; q += kPT)
+                    for(int q = tid; q < 3 * ((tp.count[l + 1] + BANK - 1) & -BANK); q += kPT)
                     {
+                        // zeros behind the last node: inverses were staged here
                         const unsigned mk = memb[o - tp.first + q / 3];
-                        const T        t  = member_sum(Rs + kRB * (mk >> 16), mk, q % 3);
+                        const T        t  = q < 3 * tp.count[l + 1]
+                                                ? member_sum(Rs + kRB * (mk >> 16), mk, q % 3)
+                                                : (T)0;
                         Rs[kRB * ((o + q / 3) / BANK) + 3 * ((o + q / 3) % BANK) + q % 3] = t;
                     }
                     __syncthreads();
@@ -724,7 +785,7 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
                     }
                     else
                     {
-                        const T* P = A.inv + (size_t)(b0 + n / BANK) * BD * BD
+                        const T* P = A.dense + (size_t)(b0 - A.first_dense + n / BANK) * BD * BD
                                      + (3 * (n % BANK) + f % 3) * BD + h;
 #pragma unroll
                         for(int u = 0; u < BD / 4; u++)
@@ -801,6 +862,7 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
         beta = k == 0 ? 0.0 : rzn / rz;
         rz   = rzn;
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load into LDS is under way
     __syncthreads();
     if(fail && tid == 0)
         A.ctl[2] = 1;  // a wait ran out
@@ -816,16 +878,14 @@ bool launch(PersistPlan& P, Mas* mas, PersistArgs<T> a, hipStream_t s)
         const MasView<T> m = mas->view<T>();
         a.vert_of_slot = m.vert_of_slot, a.bank_first = m.bank_first, a.bank_ncl = m.bank_ncl;
         a.chain = m.chain, a.child_bank = m.child_bank, a.child_mask = m.child_mask;
-        a.inv = m.inv, a.R = m.R, a.Z = m.Z, a.L = mas->levels(), a.nbank = P.banks;
+        a.inv = m.inv, a.dense = m.dense, a.R = m.R, a.Z = m.Z, a.L = mas->levels(), a.nbank = P.banks;
+        a.first_dense = mas->parts();
         a.tp = tail_plan(a.L, mas->level_sizes(), [&](int span, int levels) {
             TailPlan t;
             t.lt = a.L - levels, t.span = span;
             return persist_lds<T>(P.rows, P.halo, P.banks, t, a.L, true, a.rp2 != nullptr)
                    <= kPLds;
         });
-        // the levels below the tail use the product buffer: 64 per wave
-        if(a.tp.lt > 1 && 3 * P.rows * (a.L - a.tp.lt) < 64 * kPW)
-            return false;
     }
     const size_t fix = persist_lds<T>(P.rows, P.halo, P.banks, a.tp, a.L, MAS, a.rp2 != nullptr);
     if(fix > kPLds)
@@ -858,20 +918,21 @@ void PersistPlan::build(const Bsr& A, const std::vector<int>& part_first, hipStr
     const int G = std::min(std::min(kMaxGroups, cus), std::max(1, nb / kGroupRows));
     if(!coop || nb > kMaxRows * G)
         return;
-    // row ranges, cut at parts
+    // row ranges, cut at parts; a bank weighs as much as kBankRows rows
     const bool       mas = !part_first.empty();
     std::vector<int> rs(G + 1), bs(G + 1, 0);
     for(int g = 0; g <= G; g++)
     {
-        int r = (int)((long long)nb * g / G);
+        rs[g] = (int)((long long)nb * g / G);
         if(mas)
         {
-            bs[g] = g == G ? (int)part_first.size() - 1
-                           : (int)(std::lower_bound(part_first.begin(), part_first.end(), r)
-                                   - part_first.begin());
-            r     = part_first[bs[g]];
+            const int np = (int)part_first.size() - 1;
+            int       j  = g > 0 ? bs[g - 1] : 0;
+            while(j < np && part_first[j] + kBankRows * j < (nb + kBankRows * np) * (double)g / G)
+                j++;
+            bs[g] = j;
+            rs[g] = part_first[j];
         }
-        rs[g] = r;
     }
     int nr = 0, nh = 0, nk = 0;
     for(int g = 0; g < G; g++)

@@ -294,6 +294,28 @@ def test_pcg_one_launch_sizes(oracle, nb, pc, prec):
             assert np.linalg.norm(x - xo) <= 1e-11 * np.linalg.norm(xo)
 
 
+@pytest.mark.parametrize("nb,low", [(500, 1), (6000, 1), (43000, 3)])
+def test_pcg_one_launch_uneven_parts(oracle, nb, low):
+    """Parts of low .. 16 rows: workgroups with unequal numbers of banks, whose
+    inverses stay in LDS whole, stay there packed, or come in again each
+    iteration."""
+    import sgipc
+    A, _, b = _spd_system(oracle, nb, nb)
+    size = np.random.default_rng(1).integers(low, 17, size=nb)
+    part = np.repeat(np.arange(nb), size)[:nb].astype(np.int32)
+    for prec, bound in ((sgipc.SGIPC_MAS_FP64, 1e-11), (sgipc.SGIPC_MAS_FP32, 0.0)):
+        ls = sgipc.LinearSystem(A.rowptr, A.cols, A.vals, part, sgipc.SGIPC_PRECOND_MAS, prec)
+        x, st = ls.pcg(b, rel_tol=1e-12)
+        assert st.converged
+        assert np.linalg.norm(A.spmv(x) - b) <= 1e-10 * np.linalg.norm(b)
+        if bound:
+            x, st = ls.pcg(b, rel_tol=0.0, max_iter=13)
+            xo, _, _, _ = oracle.pcg(A, b, oracle.Mas(A, part, fp32=False), 1, rel_tol=0.0,
+                                     max_iter=13)
+            # FP64 sums in another order, amplified by at most 13 steps
+            assert np.linalg.norm(x - xo) <= bound * np.linalg.norm(xo)
+
+
 @pytest.mark.parametrize("pc", ["mas", "diag"])
 def test_pcg_beyond_one_launch(oracle, pc):
     """More rows than the one-launch solve takes (256 per workgroup): a
