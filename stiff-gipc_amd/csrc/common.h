@@ -332,6 +332,15 @@ __device__ __forceinline__ float wave_sum(float v)
     return v;
 }
 
+// Ordering of LDS between the lanes of one wave: the LDS instructions of a
+// wave execute in program order, so a compiler-only wave barrier suffices;
+// __syncthreads would also make the wave wait for its outstanding global
+// stores (workgroup-scope release).
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_wave_barrier();
+}
+
 __device__ __forceinline__ double wave_max(double v)
 {
 #pragma unroll

@@ -142,19 +142,25 @@ __device__ __forceinline__ uint32_t morton_code(double x, double y, double z)
            + expand_bits((uint32_t)z);
 }
 
-__global__ void k_morton(int n, const double* __restrict__ leaf, const double* __restrict__ scene,
-                         uint64_t* __restrict__ keys)
+// Morton code of box e's centre, then e
+__device__ __forceinline__ uint64_t morton_key(int e, const double* __restrict__ leaf,
+                                               const double* scene)
 {
-    int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if(e >= n)
-        return;
     double lo[3] = {scene[3], scene[4], scene[5]};
     double sz[3] = {scene[0] - lo[0], scene[1] - lo[1], scene[2] - lo[2]};
     double c[3];
     for(int k = 0; k < 3; k++)
         c[k] = (leaf[6 * (size_t)e + k] + leaf[6 * (size_t)e + 3 + k]) * 0.5;
     uint64_t mc = morton_code((c[0] - lo[0]) / sz[0], (c[1] - lo[1]) / sz[1], (c[2] - lo[2]) / sz[2]);
-    keys[e]     = (mc << 32) | (uint64_t)(uint32_t)e;
+    return (mc << 32) | (uint64_t)(uint32_t)e;
+}
+
+__global__ void k_morton(int n, const double* __restrict__ leaf, const double* __restrict__ scene,
+                         uint64_t* __restrict__ keys)
+{
+    int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if(e < n)
+        keys[e] = morton_key(e, leaf, scene);
 }
 
 // ------------------------------------------------------------ radix sort
@@ -277,6 +283,175 @@ __global__ void __launch_bounds__(kSortThreads) k_sort_scatter(int n, int shift,
                                + wcnt[3][threadIdx.x];
         __syncthreads();
     }
+}
+
+// The whole sort in one workgroup, for up to 1024 J keys: a pass over one digit
+// is a few microseconds of work here, against three launches of 2 to 6 us and
+// the gaps between them.  A thread holds J keys (element 64 J w + 64 j + lane in
+// the current order); ranks come from ballots and per-wave digit counters, so a
+// pass is stable, and the keys move through LDS.  What: the keys, pairs, or the
+// keys made here from the n leaf boxes (their common box into scene, Morton
+// codes; see k_box_partial, k_morton).
+enum
+{
+    SORT_KEYS  = 0,
+    SORT_PAIRS = 1,
+    SORT_BOXES = 2
+};
+constexpr int kSmallThreads = 1024;
+
+template <int J, int What>
+constexpr size_t kSmallLds = (size_t)kSmallThreads * J * (What == SORT_PAIRS ? 12 : 8)
+                             + (kSmallThreads / 64 + 1) * 256 * sizeof(unsigned);
+
+template <int J, int What>
+__global__ void __launch_bounds__(kSmallThreads)
+    k_sort_small(int n, int lo, int hi, uint64_t* __restrict__ keys, uint32_t* __restrict__ vals,
+                 const double* __restrict__ leaf, double* __restrict__ scene)
+{
+    constexpr int NW = kSmallThreads / 64;
+    extern __shared__ __align__(16) unsigned char sort_lds[];
+    uint64_t* lk    = reinterpret_cast<uint64_t*>(sort_lds);
+    unsigned* cnt   = reinterpret_cast<unsigned*>(lk + kSmallThreads * J);  // [wave][digit]
+    unsigned* dbase = cnt + 256 * NW;
+    uint32_t* lv    = dbase + 256;
+    __shared__ double   box[6][NW], sc[6];
+    __shared__ unsigned wsum[4];
+    const int t = threadIdx.x, w = t >> 6, lane = t & 63;
+    const int i0 = 64 * J * w + lane;
+    uint64_t  k[J];
+    uint32_t  v[J];
+    if constexpr(What == SORT_BOXES)
+    {
+        double b[6] = {-1e32, -1e32, -1e32, 1e32, 1e32, 1e32};
+#pragma unroll
+        for(int j = 0; j < J; j++)
+            if(i0 + 64 * j < n)
+                for(int c = 0; c < 6; c++)
+                {
+                    const double p = leaf[6 * (size_t)(i0 + 64 * j) + c];
+                    b[c] = (c < 3) ? ((b[c] < p) ? p : b[c]) : ((p < b[c]) ? p : b[c]);
+                }
+        for(int c = 0; c < 6; c++)
+        {
+            const double r = c < 3 ? wave_max(b[c]) : wave_min(b[c]);
+            if(lane == 0)
+                box[c][w] = r;
+        }
+        __syncthreads();
+        if(t < 6)
+        {
+            double r = box[t][0];
+            for(int q = 1; q < NW; q++)
+                r = (t < 3) ? ((r < box[t][q]) ? box[t][q] : r)
+                            : ((box[t][q] < r) ? box[t][q] : r);
+            scene[t] = sc[t] = r;
+        }
+        __syncthreads();
+#pragma unroll
+        for(int j = 0; j < J; j++)
+            k[j] = i0 + 64 * j < n ? morton_key(i0 + 64 * j, leaf, sc) : 0;
+    }
+    else
+    {
+#pragma unroll
+        for(int j = 0; j < J; j++)
+        {
+            const bool live = i0 + 64 * j < n;
+            k[j]            = live ? keys[i0 + 64 * j] : 0;
+            if(What == SORT_PAIRS)
+                v[j] = live ? vals[i0 + 64 * j] : 0;
+        }
+    }
+#pragma unroll 1
+    for(int sh = lo; sh < hi; sh += 8)
+    {
+        unsigned* my = cnt + 256 * w;
+        unsigned  r[J];
+        for(int q = 0; q < 4; q++)
+            my[64 * q + lane] = 0;
+        wave_lds_sync();
+#pragma unroll
+        for(int j = 0; j < J; j++)
+        {
+            const bool         live  = i0 + 64 * j < n;
+            const unsigned     d     = (unsigned)(k[j] >> sh) & 0xFF;
+            unsigned long long peers = __ballot(live);
+#pragma unroll
+            for(int b = 0; b < 8; b++)
+            {
+                const unsigned long long m = __ballot((d >> b) & 1u);
+                peers &= ((d >> b) & 1u) ? m : ~m;
+            }
+            const unsigned rank = (unsigned)__popcll(peers & ((1ull << lane) - 1ull));
+            const unsigned c    = my[d];
+            wave_lds_sync();
+            if(live && rank == 0)
+                my[d] = c + (unsigned)__popcll(peers);
+            wave_lds_sync();
+            r[j] = c + rank;
+        }
+        __syncthreads();
+        // digit t: its waves' counters become offsets; then the digits' offsets
+        unsigned tot = 0, s = 0;
+        if(t < 256)
+        {
+            unsigned c[NW];
+#pragma unroll
+            for(int q = 0; q < NW; q++)
+                c[q] = cnt[256 * q + t];
+#pragma unroll
+            for(int q = 0; q < NW; q++)
+            {
+                cnt[256 * q + t] = tot;
+                tot += c[q];
+            }
+            s = tot;
+            for(int o = 1; o < 64; o <<= 1)
+            {
+                const unsigned u = __shfl_up(s, o, 64);
+                if(lane >= o)
+                    s += u;
+            }
+            if(lane == 63)
+                wsum[w] = s;
+        }
+        __syncthreads();
+        if(t < 256)
+        {
+            for(int q = 0; q < w; q++)
+                s += wsum[q];
+            dbase[t] = s - tot;
+        }
+        __syncthreads();
+#pragma unroll
+        for(int j = 0; j < J; j++)
+            if(i0 + 64 * j < n)
+            {
+                const unsigned d   = (unsigned)(k[j] >> sh) & 0xFF;
+                const unsigned off = dbase[d] + my[d] + r[j];
+                lk[off]            = k[j];
+                if(What == SORT_PAIRS)
+                    lv[off] = v[j];
+            }
+        __syncthreads();
+#pragma unroll
+        for(int j = 0; j < J; j++)
+            if(i0 + 64 * j < n)
+            {
+                k[j] = lk[i0 + 64 * j];
+                if(What == SORT_PAIRS)
+                    v[j] = lv[i0 + 64 * j];
+            }
+    }
+#pragma unroll
+    for(int j = 0; j < J; j++)
+        if(i0 + 64 * j < n)
+        {
+            keys[i0 + 64 * j] = k[j];
+            if(What == SORT_PAIRS)
+                vals[i0 + 64 * j] = v[j];
+        }
 }
 
 // --------------------------------------------------------- Karras build
@@ -567,13 +742,38 @@ static void sort_scan(unsigned* hist, int nblk, hipStream_t s)
         scan_exclusive_u32(total, hist, hist, hist + total, s);
 }
 
+// the sort in one workgroup; false: too many keys for it.  Boxes, keys and four
+// passes: 14.5 us up to 2,048 boxes against 15 launches of together 52 us and
+// the gaps between them (a Newton iteration on a 425-vertex bar has about five
+// such sorts: 2.5 -> 2.3 ms).  Sixteen keys per thread no longer fit the
+// registers: 81 us for 14,000 boxes, 15 launches take 66 us and their gaps, and
+// the iteration was not faster; so the line lies at eight.
+template <int What>
+static bool sort_small(int n, int lo, int hi, uint64_t* keys, uint32_t* vals, const double* leaf,
+                       double* scene, hipStream_t s)
+{
+    auto go = [&](auto kern, size_t lds) {
+        hipLaunchKernelGGL(kern, dim3(1), dim3(kSmallThreads), lds, s, n, lo, hi, keys, vals, leaf,
+                           scene);
+        SG_LAUNCH_CHECK();
+        return true;
+    };
+    if(n <= 2 * kSmallThreads)
+        return go(k_sort_small<2, What>, kSmallLds<2, What>);
+    if(n <= 4 * kSmallThreads)
+        return go(k_sort_small<4, What>, kSmallLds<4, What>);
+    if(n <= 8 * kSmallThreads)
+        return go(k_sort_small<8, What>, kSmallLds<8, What>);
+    return false;
+}
+
 // stable LSD radix sort of n 64-bit keys on the 8-bit digits from bit lo to
 // bit hi (exclusive); the result ends in keys (alt: scratch of n keys, hist:
 // radix_sort_hist_size(n) counters)
 void radix_sort_keys(uint64_t* keys, uint64_t* alt, unsigned* hist, int n, int lo, int hi,
                      hipStream_t s)
 {
-    if(n <= 1)
+    if(n <= 1 || sort_small<SORT_KEYS>(n, lo, hi, keys, nullptr, nullptr, nullptr, s))
         return;
     int       nblk = (n + kSortTile - 1) / kSortTile;
     uint64_t* a    = keys;
@@ -594,7 +794,7 @@ void radix_sort_keys(uint64_t* keys, uint64_t* alt, unsigned* hist, int n, int l
 void radix_sort_pairs(uint64_t* keys, uint64_t* kalt, uint32_t* vals, uint32_t* valt,
                       unsigned* hist, int n, int lo, int hi, hipStream_t s)
 {
-    if(n <= 1)
+    if(n <= 1 || sort_small<SORT_PAIRS>(n, lo, hi, keys, vals, nullptr, nullptr, s))
         return;
     int       nblk = (n + kSortTile - 1) / kSortTile;
     uint64_t* a    = keys;
@@ -638,15 +838,20 @@ void Lbvh::build(const double* x, const double* dx, double alpha, hipStream_t s)
         return;
     hipLaunchKernelGGL(k_leaf_aabb, dim3(grid_for(n, 256)), dim3(256), 0, s, n, arity, prims, x,
                        dx, alpha, leaf.data());
-    unsigned nb = grid_for(n, 256);
-    hipLaunchKernelGGL(k_box_partial, dim3(nb), dim3(256), 0, s, n, leaf.data(), partial.data());
-    hipLaunchKernelGGL(k_box_final, dim3(1), dim3(256), 0, s, (int)nb, partial.data(), scene.data());
-    hipLaunchKernelGGL(k_morton, dim3(grid_for(n, 256)), dim3(256), 0, s, n, leaf.data(),
-                       scene.data(), keys.data());
-    SG_LAUNCH_CHECK();
     // the keys enter in index order and every pass is stable, so sorting the
     // 30 Morton bits alone orders by (morton, index)
-    radix_sort_keys(keys.data(), keys_alt.data(), hist.data(), n, 32, 62, s);
+    if(!sort_small<SORT_BOXES>(n, 32, 62, keys.data(), nullptr, leaf.data(), scene.data(), s))
+    {
+        unsigned nb = grid_for(n, 256);
+        hipLaunchKernelGGL(k_box_partial, dim3(nb), dim3(256), 0, s, n, leaf.data(),
+                           partial.data());
+        hipLaunchKernelGGL(k_box_final, dim3(1), dim3(256), 0, s, (int)nb, partial.data(),
+                           scene.data());
+        hipLaunchKernelGGL(k_morton, dim3(grid_for(n, 256)), dim3(256), 0, s, n, leaf.data(),
+                           scene.data(), keys.data());
+        SG_LAUNCH_CHECK();
+        radix_sort_keys(keys.data(), keys_alt.data(), hist.data(), n, 32, 62, s);
+    }
     hipLaunchKernelGGL(k_leaf_nodes, dim3(grid_for(n, 256)), dim3(256), 0, s, n, keys.data(),
                        nodes.data(), leaf.data(), bvs.data(), arity, prims, body, lbody.data());
     if(n > 1)

@@ -45,15 +45,6 @@ inline TailPlan tail_plan(int L, const std::vector<int>& lvl, F&& fits)
     return tp;
 }
 
-// Ordering of LDS between the lanes of one wave: the LDS instructions of a
-// wave execute in program order, so a compiler-only wave barrier suffices;
-// __syncthreads would also make the wave wait for its outstanding global
-// stores (workgroup-scope release).
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_wave_barrier();
-}
-
 // 16 bytes of T
 template <typename T>
 struct alignas(16) Vec16

@@ -132,6 +132,14 @@ def test_ccd_bound_impact(oracle):
         assert len(cg) > 0 and _key(cg) == _key(co)
 
 
+@pytest.mark.parametrize("n", [27, 38, 54])
+@pytest.mark.parametrize("which", [0, 1])
+def test_lbvh_order_sizes(oracle, n, which):
+    """trees of 1,352 to 8,533 primitives: every size class of the launch that
+    makes and sorts the keys, and the first beyond it"""
+    test_lbvh_tree_sizes(oracle, n, which)
+
+
 @pytest.mark.parametrize("n", [2, 3, 6, 9, 12, 33])
 @pytest.mark.parametrize("which", [0, 1])
 def test_lbvh_tree_sizes(oracle, n, which):

@@ -36,6 +36,19 @@ def test_vertex_keys_bit_exact(oracle, name):
     assert np.array_equal(o, oo)
 
 
+@pytest.mark.parametrize("n", [2, 64, 65, 1025, 2047, 2048, 2049, 4096, 4097, 8191, 8192, 8193])
+def test_vertex_keys_workgroup_sizes(oracle, n):
+    """sizes around the limits of the one-workgroup sort, a third of the points
+    at the same places (ties keep their order)"""
+    import sgipc
+    x = np.random.default_rng(n).random((n, 3))
+    x[n // 3:2 * (n // 3)] = x[:n // 3]
+    k, o = sgipc.spatial_sort_keys(x)
+    ko, oo = oracle.spatial_keys(x)
+    assert np.array_equal(k, ko)
+    assert np.array_equal(o, oo)
+
+
 @pytest.mark.parametrize("name", ["bar", "cubes", "hybrid"])
 def test_scene_keys_bit_exact(oracle, name):
     """vertex and tet keys of the benchmark scenes (hybrid: 983,040 bed tets
