@@ -15,11 +15,13 @@
 // tests all the way down (a leaf's box is inside its ancestors').  Proximity
 // and CCD queries skip subtrees whose primitives all belong to the query's
 // own body: such pairs are never candidates, and in scenes of many bodies
-// they are most of what a query meets.  Records are claimed with one counter
-// update per wave and event.  Bound by the dependent record loads: on 64 cubes
-// in contact (73,728 edges, 40,573 pairs) the edge-edge query takes 447 us
-// (646 us with separate node and box arrays in FP64, own-body subtrees
-// entered, and two counter updates per record).
+// they are most of what a query meets.  The leaves that a wave's walks meet
+// are collected and tested 64 at a time, whichever query they belong to.
+// Records are claimed with one counter update per wave and event.  Bound by
+// the dependent record loads of the walk.  64 cubes in contact (73,728 edges,
+// 40,573 pairs), each leaf tested where it is met / collected: edge-edge
+// 397 / 130 us, vertex-face 195 / 61 us, swept 331 / 77 and 152 / 52 us,
+// edge-triangle 226 / 116 us.
 //
 // The traversal stack lives in LDS as stk[depth][lane] (bank-conflict free),
 // its rarely reached upper part (a 64-bit-key Karras tree is at most 64 deep)
@@ -245,24 +247,34 @@ __device__ __forceinline__ float below(double x)
     return f - fmaxf(fabsf(f) * 2.4e-7f, 1e-37f);
 }
 
-// visit(sorted leaf) for every leaf whose box overlaps q within gap, until it
-// returns true.  Leaves at sorted positions up to `after` are left out: a self
-// query of the tree from its sorted leaf `after` then meets every unordered
-// pair of leaves once, from the earlier one.  qbody: skip subtrees of this
-// body (kMixedBody: none).
+// LDS of a wave's queries
+struct WaveQueries
+{
+    uint32_t stk[kStackLds][64];  // traversal stacks
+    uint32_t own[3][64];          // what a leaf visit needs of its query
+    double   q[6][64];            // query boxes
+    uint32_t item[3 * 64];        // leaves to visit: sorted leaf
+    uint8_t  of[3 * 64];          // and query (lane)
+};
+
+// visit(query lane, sorted leaf) for every leaf whose box overlaps the
+// query's box q within gap; live: this lane has a query.  Called by all lanes
+// of a wave.  The leaves that the 64 walks meet are collected and visited 64
+// at a time, one per lane and of whichever query: a visit's chain of loads
+// then holds up the wave once for 64 leaves, not once for each step in
+// which some lane met one.  A visit that returns true ends the wave's walks.
+// Leaves at sorted positions up to `after` are left out: a self query of the
+// tree from its sorted leaf `after` then meets every unordered pair of leaves
+// once, from the earlier one.  qbody: skip subtrees of this body (kMixedBody:
+// none).
 template <typename Visit>
-__device__ __forceinline__ void traverse(const Tree& T, const double* q, double gap, int qbody,
-                                         uint32_t (*stk)[64], Visit&& visit, int after = -1)
+__device__ __forceinline__ void traverse(const Tree& T, bool live, const double (&q)[6], double gap,
+                                         int qbody, WaveQueries& W, Visit&& visit, int after = -1)
 {
     const int lane = threadIdx.x;
-    if(after >= T.n - 1)
-        return;
-    if(T.n == 1)
-    {
-        if(overlap(q, T.leaf, gap))
-            visit(0);
-        return;
-    }
+#pragma unroll
+    for(int c = 0; c < 6; c++)
+        W.q[c][lane] = q[c];
     // the query box grown by gap and rounded outwards
     float ql[3], qu[3];
 #pragma unroll
@@ -278,46 +290,82 @@ __device__ __forceinline__ void traverse(const Tree& T, const double* q, double 
             ok = ok && !(h.lo[c] > qu[c]) && !(h.up[c] < ql[c]);
         return ok;
     };
+    int  n   = 0;  // collected leaves
+    auto put = [&](bool on, uint32_t leaf) {
+        const unsigned long long m = __ballot(on);
+        const int                o = n + __popcll(m & ((1ull << lane) - 1ull));
+        if(on)
+        {
+            W.item[o] = leaf & 0x7fffffffu;
+            W.of[o]   = (uint8_t)lane;
+        }
+        n += __popcll(m);
+    };
+    // the last (up to) 64 collected leaves
+    auto take = [&]() {
+        wave_lds_sync();
+        const int c  = n < 64 ? n : 64;
+        bool      ok = false;
+        if(lane < c)
+        {
+            const int s = (int)W.item[n - c + lane], o = W.of[n - c + lane];
+            double    b[6];
+#pragma unroll
+            for(int k = 0; k < 6; k++)
+                b[k] = W.q[k][o];
+            ok = overlap(b, T.leaf + 6 * (size_t)s, gap) && visit(o, s);
+        }
+        n -= c;
+        wave_lds_sync();
+        return __any(ok) != 0;
+    };
     uint32_t deep[kStackMax - kStackLds];
     int      sp   = 0;
     uint32_t node = 0;
-    bool     more = true;
-    while(more)
+    bool     more = live && T.n > 1 && after < T.n - 1;
+    if(T.n == 1)
+        put(live && after < 0, 0u);
+    while(__any(more))
     {
-        const NodeHalf L = T.rec[2 * (size_t)node], R = T.rec[2 * (size_t)node + 1];
-        const bool     hl = hit(L) && (int)(L.child & 0x7fffffffu) > after, hr = hit(R);
-        const bool     ll = L.child >> 31, lr = R.child >> 31;
-        // the next node before the leaves' visits, which the lanes then
-        // reach together
-        const bool il = hl && !ll, ir = hr && !lr;
-        if(il && ir)
+        bool     pl = false, pr = false;
+        uint32_t cl = 0, cr = 0;
+        if(more)
         {
-            if(sp < kStackLds)
-                stk[sp++][lane] = R.child;
-            else if(sp < kStackMax)
-                deep[sp++ - kStackLds] = R.child;
-        }
-        if(il || ir)
-            node = il ? L.child : R.child;
-        else if(sp == 0)
-            more = false;
-        else
-        {
-            sp--;
-            if(sp < kStackLds)
-                node = stk[sp][lane];
-            else
-                node = deep[sp - kStackLds];
-        }
-#pragma unroll 1
-        for(int h = 0; h < 2; h++)
-        {
-            const bool leaf = h == 0 ? hl && ll : hr && lr;
-            const int  s    = (int)((h == 0 ? L.child : R.child) & 0x7fffffffu);
-            if(leaf && overlap(q, T.leaf + 6 * (size_t)s, gap) && visit(s))
+            const NodeHalf L = T.rec[2 * (size_t)node], R = T.rec[2 * (size_t)node + 1];
+            const bool     hl = hit(L) && (int)(L.child & 0x7fffffffu) > after, hr = hit(R);
+            cl = L.child, cr = R.child;
+            pl = hl && (cl >> 31), pr = hr && (cr >> 31);
+            const bool il = hl && !pl, ir = hr && !pr;
+            if(il && ir)
+            {
+                if(sp < kStackLds)
+                    W.stk[sp++][lane] = cr;
+                else if(sp < kStackMax)
+                    deep[sp++ - kStackLds] = cr;
+            }
+            if(il || ir)
+                node = il ? cl : cr;
+            else if(sp == 0)
                 more = false;
+            else
+            {
+                sp--;
+                if(sp < kStackLds)
+                    node = W.stk[sp][lane];
+                else
+                    node = deep[sp - kStackLds];
+            }
         }
+        put(pl, cl);
+        put(pr, cr);
+        bool stop = false;
+        while(n >= 64 && !stop)
+            stop = take();
+        if(stop)
+            return;
     }
+    if(n > 0)
+        take();
 }
 
 __device__ __forceinline__ int query_body(int b) { return b == -1 ? kMixedBody : b; }
@@ -329,20 +377,19 @@ __global__ void __launch_bounds__(64) k_query_vf(int ns, const uint32_t* __restr
                                                  const double* __restrict__ x, Tree tree,
                                                  double dHat, PairSink sk)
 {
-    __shared__ uint32_t stk[kStackLds][64];
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i < ns)
-    {
-        int    v    = (int)surf[i];
-        double q[6] = {x[3 * v], x[3 * v + 1], x[3 * v + 2], x[3 * v], x[3 * v + 1], x[3 * v + 2]};
-        double gap  = sqrt(dHat);
-        traverse(tree, q, gap, query_body(body[v]), stk, [&](int s) {
-            uint3 f = faces[tree.element(s)];
-            if(vf_ok(body, bt, v, f))
-                check_pt(x, v, f.x, f.y, f.z, dHat, sk);
-            return false;
-        });
-    }
+    __shared__ WaveQueries W;
+    const int  i    = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool live = i < ns;
+    const int  v    = (int)surf[live ? i : 0];
+    const double q[6] = {x[3 * v], x[3 * v + 1], x[3 * v + 2], x[3 * v], x[3 * v + 1], x[3 * v + 2]};
+    W.own[0][threadIdx.x] = (uint32_t)v;
+    traverse(tree, live, q, sqrt(dHat), query_body(body[v]), W, [&](int o, int s) {
+        const int v = (int)W.own[0][o];
+        uint3     f = faces[tree.element(s)];
+        if(vf_ok(body, bt, v, f))
+            check_pt(x, v, f.x, f.y, f.z, dHat, sk);
+        return false;
+    });
     sk.flush();
 }
 
@@ -356,30 +403,33 @@ __global__ void __launch_bounds__(64) k_query_ee(int ne, const uint2* __restrict
                                                  const double* __restrict__ xr, Tree tree,
                                                  double dHat, PairSink sk)
 {
-    __shared__ uint32_t stk[kStackLds][64];
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i < ne)
-    {
-        int    self = (int)tree.element(i);
-        double q[6];
-        for(int c = 0; c < 6; c++)
-            q[c] = tree.leaf[6 * (size_t)i + c];
-        uint2  e   = edges[self];
-        double gap = sqrt(dHat);
-        traverse(
-            tree, q, gap, query_body(body[e.x]), stk,
-            [&](int s) {
-                const int obj = (int)tree.element(s);
-                const int lo  = self < obj ? self : obj;
-                const int hi  = self < obj ? obj : self;
-                uint2     o   = edges[obj];
-                uint2     a = lo == self ? e : o, b = lo == self ? o : e;
-                if(ee_ok(body, bt, a, b, lo, hi))
-                    check_ee(x, xr, a.x, a.y, b.x, b.y, hi, dHat, sk);
-                return false;
-            },
-            i);
-    }
+    __shared__ WaveQueries W;
+    const int  i    = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool live = i < ne;
+    const int  il   = live ? i : 0;
+    const int  self = (int)tree.element(il);
+    double     q[6];
+    for(int c = 0; c < 6; c++)
+        q[c] = tree.leaf[6 * (size_t)il + c];
+    const uint2 e = edges[self];
+    W.own[0][threadIdx.x] = (uint32_t)self;
+    W.own[1][threadIdx.x] = e.x;
+    W.own[2][threadIdx.x] = e.y;
+    traverse(
+        tree, live, q, sqrt(dHat), query_body(body[e.x]), W,
+        [&](int p, int s) {
+            const int   self = (int)W.own[0][p];
+            const uint2 e    = make_uint2(W.own[1][p], W.own[2][p]);
+            const int   obj  = (int)tree.element(s);
+            const int   lo   = self < obj ? self : obj;
+            const int   hi   = self < obj ? obj : self;
+            const uint2 o    = edges[obj];
+            const uint2 a = lo == self ? e : o, b = lo == self ? o : e;
+            if(ee_ok(body, bt, a, b, lo, hi))
+                check_ee(x, xr, a.x, a.y, b.x, b.y, hi, dHat, sk);
+            return false;
+        },
+        i);
     sk.flush();
 }
 
@@ -409,21 +459,21 @@ __global__ void __launch_bounds__(64) k_ccd_vf(int ns, const uint32_t* __restric
                                                const double* __restrict__ dx, double alpha,
                                                Tree tree, double dHat, CandSink sk)
 {
-    __shared__ uint32_t stk[kStackLds][64];
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i >= ns)
-        return;
-    int    v = (int)surf[i];
-    double q[6];
+    __shared__ WaveQueries W;
+    const int  i    = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool live = i < ns;
+    const int  v    = (int)surf[live ? i : 0];
+    double     q[6];
     for(int c = 0; c < 3; c++)
     {
         double a = x[3 * v + c], b = x[3 * v + c] - dx[3 * v + c] * alpha;
         q[c]     = (a < b) ? b : a;   // upper: combines(v - dx alpha) after (v, v)
         q[3 + c] = (b < a) ? b : a;
     }
-    double gap = sqrt(dHat);
-    traverse(tree, q, gap, query_body(body[v]), stk, [&](int s) {
-        uint3 f = faces[tree.element(s)];
+    W.own[0][threadIdx.x] = (uint32_t)v;
+    traverse(tree, live, q, sqrt(dHat), query_body(body[v]), W, [&](int o, int s) {
+        const int v = (int)W.own[0][o];
+        uint3     f = faces[tree.element(s)];
         if(((body[v] != body[f.x]) || (body[v] == -1))
            && !(bt[v] >= 2 && bt[f.x] >= 2 && bt[f.y] >= 2 && bt[f.z] >= 2)
            && v != (int)f.x && v != (int)f.y && v != (int)f.z)
@@ -437,24 +487,28 @@ __global__ void __launch_bounds__(64) k_ccd_ee(int ne, const uint2* __restrict__
                                                const int* __restrict__ bt, Tree tree, double dHat,
                                                CandSink sk)
 {
-    __shared__ uint32_t stk[kStackLds][64];
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i >= ne)
-        return;
-    int    self = (int)tree.element(i);
-    double q[6];
+    __shared__ WaveQueries W;
+    const int  i    = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool live = i < ne;
+    const int  il   = live ? i : 0;
+    const int  self = (int)tree.element(il);
+    double     q[6];
     for(int c = 0; c < 6; c++)
-        q[c] = tree.leaf[6 * (size_t)i + c];
-    uint2  e   = edges[self];
-    double gap = sqrt(dHat);
+        q[c] = tree.leaf[6 * (size_t)il + c];
+    const uint2 e = edges[self];
+    W.own[0][threadIdx.x] = (uint32_t)self;
+    W.own[1][threadIdx.x] = e.x;
+    W.own[2][threadIdx.x] = e.y;
     traverse(
-        tree, q, gap, query_body(body[e.x]), stk,
-        [&](int s) {
-            const int obj = (int)tree.element(s);
-            const int lo  = self < obj ? self : obj;
-            const int hi  = self < obj ? obj : self;
-            uint2     o   = edges[obj];
-            uint2     a = lo == self ? e : o, b = lo == self ? o : e;
+        tree, live, q, sqrt(dHat), query_body(body[e.x]), W,
+        [&](int p, int s) {
+            const int   self = (int)W.own[0][p];
+            const uint2 e    = make_uint2(W.own[1][p], W.own[2][p]);
+            const int   obj  = (int)tree.element(s);
+            const int   lo   = self < obj ? self : obj;
+            const int   hi   = self < obj ? obj : self;
+            const uint2 o    = edges[obj];
+            const uint2 a = lo == self ? e : o, b = lo == self ? o : e;
             if(ee_ok(body, bt, a, b, lo, hi))
                 sk.emit(make_int4(a.x, a.y, b.x, b.y));
             return false;
@@ -490,27 +544,30 @@ __global__ void __launch_bounds__(64) k_edge_tri(int nf, const uint3* __restrict
                                                  const double* __restrict__ x, Tree ftree,
                                                  Tree tree, int* hit)
 {
-    __shared__ uint32_t stk[kStackLds][64];
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i >= nf)
-        return;
-    uint3  F = faces[ftree.element(i)];
-    double q[6];
+    __shared__ WaveQueries W;
+    const int  i    = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool live = i < nf;
+    const int  il   = live ? i : 0;
+    const uint3 f   = faces[ftree.element(il)];
+    double      q[6];
     for(int c = 0; c < 6; c++)
-        q[c] = ftree.leaf[6 * (size_t)i + c];
-    bool found = false;
-    traverse(tree, q, 0.0, kMixedBody, stk, [&](int s) {
-        uint2 E = edges[tree.element(s)];
+        q[c] = ftree.leaf[6 * (size_t)il + c];
+    W.own[0][threadIdx.x] = f.x;
+    W.own[1][threadIdx.x] = f.y;
+    W.own[2][threadIdx.x] = f.z;
+    traverse(tree, live, q, 0.0, kMixedBody, W, [&](int o, int s) {
+        const uint3 F = make_uint3(W.own[0][o], W.own[1][o], W.own[2][o]);
+        const uint2 E = edges[tree.element(s)];
         if(F.x == E.x || F.x == E.y || F.y == E.x || F.y == E.y || F.z == E.x || F.z == E.y)
             return false;
         if(bt[F.x] >= 2 && bt[F.y] >= 2 && bt[F.z] >= 2 && bt[E.x] >= 2 && bt[E.y] >= 2)
             return false;
-        found = seg_tri(ld3(x + 3 * E.x), ld3(x + 3 * E.y), ld3(x + 3 * F.x), ld3(x + 3 * F.y),
-                        ld3(x + 3 * F.z));
+        const bool found = seg_tri(ld3(x + 3 * E.x), ld3(x + 3 * E.y), ld3(x + 3 * F.x),
+                                   ld3(x + 3 * F.y), ld3(x + 3 * F.z));
+        if(found)
+            atomicExch(hit, 1);
         return found;
     });
-    if(found)
-        atomicExch(hit, 1);
 }
 
 __global__ void k_ground_intersect(const unsigned* __restrict__ gcount,

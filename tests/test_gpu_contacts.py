@@ -159,6 +159,26 @@ def test_lbvh_tree_sizes(oracle, n, which):
     np.testing.assert_array_equal(bv.view(np.uint64), bvo.view(np.uint64))
 
 
+@pytest.mark.parametrize("cells,dhat", [(1, 0.02), (1, 0.1), (2, 0.05), (3, 0.03)])
+def test_contacts_many_leaves(oracle, cells, dhat):
+    """two cubes and a contact distance of up to their size: from fewer queries
+    than a wave has lanes to walks that meet most leaves of the tree; the pairs
+    of the brute-force search"""
+    import sgipc
+    from sgipc import scene as S
+    sc = S.stack_scene(n=2, cells=cells, size=0.1, gap=0.01, dhat=dhat)
+    sc.body_id = np.full_like(sc.body_id, -1)
+    x = sc.x + 1e-4 * np.random.default_rng(cells).normal(size=sc.x.shape)
+    sim = sgipc.Simulation(sc)
+    sim.set_positions(x)
+    pairs, counts, _ = sim.contacts(cap=100000)
+    pb, cb = oracle.contact_pairs(sc, x, "brute", cap=100000)
+    key = lambda p: sorted(map(tuple, np.asarray(p).tolist()))
+    print(f"[contact-leaves] cells={cells} dhat={dhat} pairs={counts.tolist()}", flush=True)
+    assert counts[0] > 0 and key(pairs) == key(pb)
+    np.testing.assert_array_equal(counts, cb)
+
+
 @pytest.mark.parametrize("ids", ["distinct", "same", "none", "mixed"])
 def test_contacts_by_body_id(oracle, ids):
     """four cubes within a large contact distance, their vertices of distinct
