@@ -12,8 +12,9 @@
 // arriving at the second one and waiting for it; LDS left over keeps the
 // inverse rows of the tail products and level-0 inverses.  Per iteration, a
 // launch per operation against this: 24.2 / 13.1 us on 425 rows, 18 / 8.5 us on
-// 7,560 (block Jacobi), 25.7 / 13.5 us on 6,480 (FP64 MAS), 38.4 / 23.3 us on
-// 46,656 (where streaming the inverses, 9 KB per 16 rows, takes a quarter).
+// 7,560 (block Jacobi), 25.7 / 13.5 us on 6,480 (FP64 MAS), 38.4 / 21.4 us on
+// 46,656 (where the barriers take half, and the level-0 products and the
+// tail's R, which every workgroup reads and restricts whole, most of the rest).
 //
 // Exchange between workgroups: only z (read back by the neighbours' halos),
 // the coarse R and Z, and, for contact columns, p; at check iterations x.
@@ -57,7 +58,7 @@ constexpr int kMaxGroups = 256;
 constexpr int kGroupRows = 64;
 // Rows that a level-0 bank counts for when the rows are shared out: the waves
 // take one bank product each at a time, and banks hold 3 .. 16 rows.  By rows
-// alone the workgroups of a 43,264-row system get up to 25 banks, 17 on
+// alone the workgroups of a 46,656-row system get up to 25 banks, 17 on
 // average, and wait for the largest; with 8 rows per bank up to 22
 constexpr int kBankRows  = 8;
 constexpr int kSlotWords = 4;              // two doubles in four words
@@ -401,7 +402,7 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
     // The inverses that found no place for the whole solve come into the
     // tail's buffers, which are free until level 0 is done, while the
     // workgroup waits at a barrier. 1 KB per wave and step; a step that would
-    // end beyond the last bank starts earlier.  43,264 rows, an iteration: 24.6
+    // end beyond the last bank starts earlier.  46,656 rows, an iteration: 24.6
     // us with these banks read where they are used, 21.4 us (with kBankRows).
     auto load_stage = [&]() {
         if constexpr(MAS)
