@@ -210,8 +210,11 @@ __global__ void __launch_bounds__(1024) k_scan_banks(int level, int total_map, i
     }
 }
 
-// new (level l+1) local ids, goingNext and per-bank first/count
-__global__ void __launch_bounds__(256) k_assign(int level, int total_map, const int* __restrict__ lvl,
+// new (level l+1) local ids, goingNext and per-bank first/count; has_next: level
+// l+1 is a level of the hierarchy (the members of the nodes above the last one
+// have no entries in child_bank and child_mask)
+__global__ void __launch_bounds__(256) k_assign(int level, int has_next, int total_map,
+                                                const int* __restrict__ lvl,
                                                 const int* __restrict__ vert_of_slot,
                                                 const unsigned* __restrict__ comp,
                                                 const int* __restrict__ bank_prefix,
@@ -252,8 +255,11 @@ __global__ void __launch_bounds__(256) k_assign(int level, int total_map, const 
     going_next[off_l + t] = off_n + id;
     // the bank holding the members of the new node and their lanes in it
     // (every member stores the same values)
-    child_bank[off_n + id] = (off_l >> 4) + bank;
-    child_mask[off_n + id] = c;
+    if(has_next)
+    {
+        child_bank[off_n + id] = (off_l >> 4) + bank;
+        child_mask[off_n + id] = c;
+    }
 }
 
 // per fine vertex: node id at level l+1 and its chain entry
@@ -906,6 +912,7 @@ void Mas::init(const Bsr& A, const int* part_id, const MasConfig& cfg, hipStream
     node_.resize((size_t)L_ * nv_);
     chain_.resize((size_t)nv_ * (L_ > 1 ? L_ - 1 : 1));
     lvl_.resize(2 * (L_ + 2));
+    // nodes of L_ levels, none larger than level 0 (as large where nothing clusters)
     size_t bound = (size_t)L_ * (total_map_ + BANK) + BANK;
     going_next_.resize(bound);
     child_bank_.resize(bound);
@@ -928,8 +935,8 @@ void Mas::cluster_level(int level, hipStream_t s)
     hipLaunchKernelGGL(k_scan_banks, dim3(1), dim3(1024), 0, s, level, total_map_, lvl_.data(),
                        bank_cnt_.data(), bank_prefix_.data());
     SG_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_assign, dim3(g), dim3(256), 0, s, level, total_map_, lvl_.data(),
-                       vert_of_slot_.data(), comp_.data(), bank_prefix_.data(), bank_cnt_.data(),
+    hipLaunchKernelGGL(k_assign, dim3(g), dim3(256), 0, s, level, level + 1 < L_ ? 1 : 0,
+                       total_map_, lvl_.data(), vert_of_slot_.data(), comp_.data(), bank_prefix_.data(), bank_cnt_.data(),
                        newid_.data(), going_next_.data(), bank_first_.data(), bank_ncl_.data(),
                        child_bank_.data(), child_mask_.data());
     SG_LAUNCH_CHECK();

@@ -241,6 +241,35 @@ def test_mas_apply_workgroup_edges(oracle, nb, kind, prec):
     assert rel(ls.precond(r), m.apply(r)) < (2e-5 if fp32 else 1e-10)
 
 
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("nb", [2000, 3000, 5000, 20000])
+def test_mas_nothing_clusters(oracle, nb, prec):
+    """Blocks without couplings: every level has as many nodes as there are
+    vertices, the most that the hierarchy's arrays have to hold.  The apply is
+    the inverse block once per level."""
+    import sgipc
+    rng = np.random.default_rng(nb)
+    S = rng.normal(size=(nb, 3, 3))
+    D = 2.0 * np.eye(3) + 0.1 * S @ S.transpose(0, 2, 1)
+    fp32 = prec == "fp32"
+    part = (np.arange(nb) // 16).astype(np.int32)
+    ls = sgipc.LinearSystem(np.arange(nb + 1), np.arange(nb), D, part, sgipc.SGIPC_PRECOND_MAS,
+                            sgipc.SGIPC_MAS_FP32 if fp32 else sgipc.SGIPC_MAS_FP64)
+    L, sizes, total = ls.mas_info()
+    print(f"[mas-uncoupled] nb={nb} {prec} levels={L} sizes={sizes.tolist()}", flush=True)
+    pad = (nb + 15) // 16 * 16
+    assert sizes[1:, 0].tolist() == [nb] * L and total == L * pad
+    np.testing.assert_array_equal(ls.mas_chain().reshape(nb, L - 1),
+                                  np.arange(nb)[:, None] + pad * np.arange(1, L))
+    r = rng.normal(size=3 * nb)
+    x = np.linalg.solve(D, r.reshape(-1, 3, 1)).ravel()
+    # the blocks' condition is a few; L terms rounded at the inverses' precision
+    bound = 1e-6 if fp32 else 1e-14
+    assert rel(ls.precond(r), L * x) < bound
+    # so the first iteration of a solve (max_iter is one more) ends at the solution
+    assert rel(ls.pcg(r, rel_tol=0.0, max_iter=2)[0], x) < bound
+
+
 def _spd_system(oracle, nb, seed, reach=40):
     """A diagonally dominant block system with couplings to the next rows and
     to random far ones (rows of 3 to about 20 blocks), 16-row parts."""
