@@ -57,7 +57,7 @@ typedef struct sgipc_pcg_stats {
     int32_t iterations;       /* PCG iterations (reference count semantics)    */
     int32_t outer_iterations; /* 1; 2 when the mixed solve fell back to FP64    */
     int32_t converged;
-    int32_t pad;
+    int32_t one_launch;       /* 1: the FP64 solve ran as one launch            */
     double  rel_residual;     /* ||b - A x||_2 / ||b||_2 recomputed in FP64    */
     double  rz0, rz;          /* preconditioned residual norms (last sweep)    */
     double  ms;               /* device time of the solve                      */
@@ -115,6 +115,12 @@ int sgipc_mm_read_vector(const char* path, double* b, int32_t cap, int32_t* m);
 /* work of the system on the caller's stream from now on (hipStream_t;
  * NULL returns to the system's own stream) */
 int sgipc_ls_set_stream(sgipc_ls_t ls, void* stream);
+/* FP64 solves of up to 65,536 block rows (a system without affine bodies, or
+ * with MAS) whose row ranges fit the compute units run as one launch, in which
+ * workgroups wait for each other at grid barriers.  polls: the most polls of
+ * such a wait, 0 to run a launch per operation instead, -1 for the default.
+ * sgipc_pcg_stats.one_launch tells which way a solve ran. */
+int sgipc_ls_one_launch(sgipc_ls_t ls, int32_t polls);
 
 /* sgipc_ls_pcg without allocating.  No counterpart in the reference: it is for
  * callers that cannot allocate device memory (code under HIP graph capture,
@@ -250,6 +256,8 @@ int sgipc_mm_export_step(sgipc_t ctx, const char* dir, int32_t frame);
  * NULL returns to the context's own stream).  The reference runs on the
  * per-thread default stream. */
 int sgipc_set_stream(sgipc_t ctx, void* stream);
+/* sgipc_ls_one_launch for the context's linear solves */
+int sgipc_one_launch(sgipc_t ctx, int32_t polls);
 
 /* Step-size bounds of a vertex direction dx [3 n_verts] at the current
  * positions (x_new = x - alpha dx; solve_subIP, GIPC.cu:10786-10822):

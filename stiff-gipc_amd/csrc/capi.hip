@@ -192,6 +192,14 @@ int sgipc_ls_set_stream(sgipc_ls_t ls, void* stream)
     });
 }
 
+int sgipc_ls_one_launch(sgipc_ls_t ls, int32_t polls)
+{
+    return guard([&] {
+        SG_CHECK(ls, SGIPC_EINVAL, "null system");
+        ls->plan.set_polls(polls);
+    });
+}
+
 int sgipc_ls_destroy(sgipc_ls_t ls)
 {
     return guard([&] { delete ls; });
@@ -263,6 +271,7 @@ int sgipc_ls_pcg(sgipc_ls_t ls, const double* b, double* x, const sgipc_pcg_cfg*
             stats->iterations       = st.iterations;
             stats->outer_iterations = st.outer_iterations;
             stats->converged        = st.converged ? 1 : 0;
+            stats->one_launch       = st.one_launch ? 1 : 0;
             stats->rel_residual     = st.rel_residual;
             stats->rz0              = st.rz0;
             stats->rz               = st.rz;
@@ -499,6 +508,11 @@ int sgipc_step_log(sgipc_t ctx, sgipc_iter_stats* out, int32_t cap, int32_t* n)
 int sgipc_set_stream(sgipc_t ctx, void* stream)
 {
     return guard([&] { ctx_of(ctx).set_stream(static_cast<hipStream_t>(stream)); });
+}
+
+int sgipc_one_launch(sgipc_t ctx, int32_t polls)
+{
+    return guard([&] { ctx_of(ctx).set_one_launch(polls); });
 }
 
 int sgipc_ccd_bound(sgipc_t h, const double* dx, double* out)

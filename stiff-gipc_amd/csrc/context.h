@@ -39,6 +39,7 @@ class Context
     const std::vector<sgipc_iter_stats>& step_log() const { return step_log_; }
     // the caller's stream (nullptr: the context's own)
     void   set_stream(hipStream_t s);
+    void   set_one_launch(int polls) { plan_.set_polls(polls); }
     double animation_rate() const { return dev_.soft_rate; }
 
     // hot-path pieces exposed through the C ABI

@@ -289,6 +289,7 @@ struct PcgStats
     int    outer_iterations = 0;  // 1, or 2 when the mixed mode fell back to FP64
     int    breakdown        = 0;  // 1 non-finite r.z, 2 diverged (mixed mode)
     bool   converged        = false;
+    bool   one_launch       = false;  // the FP64 solve ran as one launch (persist.hip)
     bool   stalled          = false;  // mixed mode: FP32 iteration stopped making progress
     double rz0 = 0, rz = 0;
     double rel_residual = 0;

@@ -1078,7 +1078,8 @@ PcgStats Pcg::solve_t(const SysView& S, Precond pc, Mas* mas, const V* b, V* x,
                              W.z.data(), W.p[0].data(), W.p[1].data(), cfg, maxit, every, &pr, s))
             {
                 PcgStats st;
-                st.rz0 = pr.rz0;
+                st.one_launch = true;
+                st.rz0        = pr.rz0;
                 if(pr.rz0 == 0.0 || !(pr.rz0 == pr.rz0))
                 {
                     st.converged = (pr.rz0 == 0.0);

@@ -106,6 +106,7 @@ int sgipc_ls_pcg_noalloc(sgipc_ls_t ls, const double* b, double* x, const sgipc_
             stats->iterations       = st.iterations;
             stats->outer_iterations = st.outer_iterations;
             stats->converged        = st.converged ? 1 : 0;
+            stats->one_launch       = st.one_launch ? 1 : 0;
             stats->rel_residual     = st.rel_residual;
             stats->rz0              = st.rz0;
             stats->rz               = st.rz;

@@ -17,7 +17,17 @@ class PersistPlan
     // part_first: first row of each MAS part (size parts + 1), empty for the
     // block-Jacobi preconditioner
     void build(const Bsr& A, const std::vector<int>& part_first, hipStream_t s);
-    bool ready() const { return groups > 0; }
+    bool ready() const { return groups > 0 && polls != 0; }
+    // most polls of a wait at a grid barrier; 0: not this way, -1: the default
+    void set_polls(int n)
+    {
+        SG_CHECK(n >= -1, -1, "the number of polls is -1, 0 or positive");
+        polls = n < 0 ? kPolls : n;
+    }
+
+    // some seconds
+    static constexpr int kPolls = 1 << 22;
+    int polls = kPolls;
 
     int groups = 0;                            // workgroups (0: not this way)
     int rows = 0, halo = 0, banks = 0;         // most of one workgroup

@@ -62,7 +62,6 @@ constexpr int kGroupRows = 64;
 // average, and wait for the largest; with 8 rows per bank up to 22
 constexpr int kBankRows  = 8;
 constexpr int kSlotWords = 4;              // two doubles in four words
-constexpr int kMaxPolls  = 1 << 22;
 // R of a 16-node bank in LDS takes 50 entries instead of 48: the members of
 // consecutive clusters lie in consecutive banks, and 48 would put their reads
 // on the same LDS banks
@@ -109,12 +108,13 @@ struct PersistArgs
     u64*    slots;
     int*    ctl;
     double* out;
+    int     polls;
 };
 
 struct Barrier
 {
     u64*     slots;
-    int      groups, b;
+    int      groups, b, polls;
     unsigned epoch = 0;
     double * part, *tot;  // LDS: 2 kPW each
     int*     fail;        // LDS
@@ -165,7 +165,7 @@ struct Barrier
             constexpr int M  = N > 0 ? 2 * N : 1;
             const u64*    w8 = words(threadIdx.x);
             u64           q[M];
-            int           polls = 0;
+            int           n = 0;
             bool          there;
             do
             {
@@ -176,7 +176,7 @@ struct Barrier
 #pragma unroll
                 for(int i = 0; i < M; i++)
                     there = there && (unsigned)q[i] == epoch;
-            } while(!there && ++polls < kMaxPolls);
+            } while(!there && ++n < polls);
             if(!there)
                 *fail = 1;
             if(N > 0)
@@ -290,7 +290,7 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
     const int v0 = A.rstart[b], nloc = A.rstart[b + 1] - v0;
     const int h0 = A.hptr[b], nh = A.hptr[b + 1] - h0;
     const int n3 = 3 * nloc;
-    Barrier   bar{A.slots, A.groups, b, 0u, bar_part, bar_tot, &fail};
+    Barrier   bar{A.slots, A.groups, b, A.polls, 0u, bar_part, bar_tot, &fail};
     if(tid == 0)
         fail = 0;
 
@@ -1006,7 +1006,7 @@ bool persist_solve(PersistPlan& P, const SysView& S, Mas* mas, const double* din
         a.b = b, a.x = x, a.z = z, a.p0 = p0, a.p1 = p1, a.dinv = dinv;
         a.rel2 = cfg.rel_tol * cfg.rel_tol, a.abs2 = cfg.abs_tol * cfg.abs_tol;
         a.q_ref = cfg.q_ref, a.use_rz = cfg.use_rz ? 1 : 0, a.maxit = maxit, a.every = every;
-        a.slots = P.slots.data(), a.ctl = P.ctl.data(), a.out = P.out.data();
+        a.slots = P.slots.data(), a.ctl = P.ctl.data(), a.out = P.out.data(), a.polls = P.polls;
         return launch<T, MAS>(P, mas, a, s);
     };
     SG_HIP(hipMemsetAsync(P.slots.data(), 0, P.slots.size() * sizeof(u64), s));

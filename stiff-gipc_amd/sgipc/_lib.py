@@ -36,8 +36,8 @@ class PcgCfg(C.Structure):
 
 class PcgStats(C.Structure):
     _fields_ = [("iterations", C.c_int32), ("outer_iterations", C.c_int32),
-                ("converged", C.c_int32), ("pad", C.c_int32), ("rel_residual", C.c_double),
-                ("rz0", C.c_double), ("rz", C.c_double), ("ms", C.c_double)]
+                ("converged", C.c_int32), ("one_launch", C.c_int32),
+                ("rel_residual", C.c_double), ("rz0", C.c_double), ("rz", C.c_double), ("ms", C.c_double)]
 
 
 class IterStats(C.Structure):
@@ -94,6 +94,7 @@ EXPORTS = [
     "sgipc_ls_create_bcoo", "sgipc_ls_create_mm", "sgipc_ls_block_rows", "sgipc_mm_read_vector",
     "sgipc_mm_read_upper_bcoo", "sgipc_ls_set_stream", "sgipc_set_dof_order", "sgipc_mm_export",
     "sgipc_set_stream", "sgipc_mm_export_step", "sgipc_step_log", "sgipc_spatial_sort_keys",
+    "sgipc_ls_one_launch", "sgipc_one_launch",
 ]
 SGIPC_DOF_FEM_FIRST = 0
 SGIPC_DOF_ABD_FIRST = 1
@@ -128,6 +129,7 @@ def lib():
         L.sgipc_mm_read_upper_bcoo.argtypes = [C.c_char_p, ip, ip, ip, ip, dp, C.c_int32]
         L.sgipc_spatial_sort_keys.argtypes = [C.c_int32, dp, C.c_int32, up, C.c_int32, u64p, up]
         L.sgipc_ls_set_stream.argtypes = [C.c_void_p, C.c_void_p]
+        L.sgipc_ls_one_launch.argtypes = [C.c_void_p, C.c_int32]
         if hasattr(L, "sgipc_create"):
             L.sgipc_create.argtypes = [C.POINTER(SceneDesc), C.POINTER(C.c_void_p)]
             L.sgipc_destroy.argtypes = [C.c_void_p]
@@ -146,6 +148,7 @@ def lib():
             L.sgipc_set_dof_order.argtypes = [C.c_void_p, C.c_int32]
             L.sgipc_mm_export.argtypes = [C.c_void_p, C.c_char_p, C.c_int32, C.c_int32]
             L.sgipc_set_stream.argtypes = [C.c_void_p, C.c_void_p]
+            L.sgipc_one_launch.argtypes = [C.c_void_p, C.c_int32]
             L.sgipc_mm_export_step.argtypes = [C.c_void_p, C.c_char_p, C.c_int32]
             L.sgipc_step_log.argtypes = [C.c_void_p, C.POINTER(IterStats), C.c_int32,
                                          C.POINTER(C.c_int32)]
@@ -316,6 +319,11 @@ class LinearSystem:
         check(lib().sgipc_ls_pcg_noalloc(self.h, P(np.ascontiguousarray(b, np.float64)), P(x),
                                          C.byref(cfg), C.byref(st)))
         return x, st
+
+    def one_launch(self, polls=-1):
+        """how FP64 solves run: 0 a launch per operation, -1 as one launch where
+        the system allows it, n > 0 the same with at most n polls in a wait"""
+        check(lib().sgipc_ls_one_launch(self.h, int(polls)))
 
     def mas_info(self):
         L = C.c_int32()
@@ -506,6 +514,10 @@ class Simulation:
                 solver_precision=SGIPC_SOLVE_FP64):
         cfg = PcgCfg(rel_tol, abs_tol, max_iter, int(use_rz), check_every, solver_precision)
         check(lib().sgipc_set_pcg(self.h, C.byref(cfg)))
+
+    def one_launch(self, polls=-1):
+        """how FP64 solves run (LinearSystem.one_launch)"""
+        check(lib().sgipc_one_launch(self.h, int(polls)))
 
     def profile(self, every=1):
         """Time every `every`-th launch of each profiled kernel (0: off)."""

@@ -308,7 +308,7 @@ def test_pcg_one_launch_sizes(oracle, nb, pc, prec):
         x, st = ls.pcg(b, rel_tol=1e-12, use_rz=use_rz)
         print(f"[one-launch] nb={nb} {pc} {prec} rz={use_rz} it={st.iterations} "
               f"relres={st.rel_residual:.2e}", flush=True)
-        assert st.converged and st.iterations % 10 == 0
+        assert st.converged and st.iterations % 10 == 0 and st.one_launch == 1
         # the residual norm follows the tested norm up to the conditioning
         # (about 10) of the preconditioned system
         assert np.linalg.norm(A.spmv(x) - b) <= 1e-10 * np.linalg.norm(b)
@@ -318,7 +318,7 @@ def test_pcg_one_launch_sizes(oracle, nb, pc, prec):
             x, st = ls.pcg(b, rel_tol=0.0, max_iter=cap)
             xo, ito, _, _ = oracle.pcg(A, b, m, 1 if pc == "mas" else 0, rel_tol=0.0,
                                        max_iter=cap)
-            assert st.iterations == ito == cap and not st.converged
+            assert st.iterations == ito == cap and not st.converged and st.one_launch == 1
             # FP64 sums in another order, amplified by at most cap steps
             assert np.linalg.norm(x - xo) <= 1e-11 * np.linalg.norm(xo)
 
@@ -335,7 +335,7 @@ def test_pcg_one_launch_uneven_parts(oracle, nb, low):
     for prec, bound in ((sgipc.SGIPC_MAS_FP64, 1e-11), (sgipc.SGIPC_MAS_FP32, 0.0)):
         ls = sgipc.LinearSystem(A.rowptr, A.cols, A.vals, part, sgipc.SGIPC_PRECOND_MAS, prec)
         x, st = ls.pcg(b, rel_tol=1e-12)
-        assert st.converged
+        assert st.converged and st.one_launch == 1
         assert np.linalg.norm(A.spmv(x) - b) <= 1e-10 * np.linalg.norm(b)
         if bound:
             x, st = ls.pcg(b, rel_tol=0.0, max_iter=13)
@@ -355,9 +355,41 @@ def test_pcg_beyond_one_launch(oracle, pc):
                             sgipc.SGIPC_PRECOND_MAS if pc == "mas" else sgipc.SGIPC_PRECOND_DIAG,
                             sgipc.SGIPC_MAS_FP64)
     x, st = ls.pcg(b, rel_tol=1e-12)
-    assert st.converged
+    assert st.converged and st.one_launch == 0
     assert np.linalg.norm(A.spmv(x) - b) <= 1e-10 * np.linalg.norm(b)
     m = oracle.Mas(A, part, fp32=False) if pc == "mas" else None
     x, st = ls.pcg(b, rel_tol=0.0, max_iter=13)
     xo, _, _, _ = oracle.pcg(A, b, m, 1 if pc == "mas" else 0, rel_tol=0.0, max_iter=13)
     assert np.linalg.norm(x - xo) <= 1e-11 * np.linalg.norm(xo)
+
+
+@pytest.mark.parametrize("noalloc", [False, True])
+@pytest.mark.parametrize("pc,prec", [("mas", "fp32"), ("mas", "fp64"), ("diag", "fp64")])
+@pytest.mark.parametrize("nb", [40, 700, 8200])
+def test_pcg_ways_agree(oracle, nb, pc, prec, noalloc):
+    """A solve as one launch and as a launch per operation, chosen by the
+    caller: the stats say which way it ran, the counts are equal, and after
+    three iterations, well before convergence hides the preconditioner, the
+    iterates differ by rounding."""
+    import sgipc
+    A, part, b = _spd_system(oracle, nb, nb)
+    ls = sgipc.LinearSystem(A.rowptr, A.cols, A.vals, part,
+                            sgipc.SGIPC_PRECOND_MAS if pc == "mas" else sgipc.SGIPC_PRECOND_DIAG,
+                            sgipc.SGIPC_MAS_FP32 if prec == "fp32" else sgipc.SGIPC_MAS_FP64)
+    pcg = ls.pcg_noalloc if noalloc else ls.pcg
+    runs = []
+    for polls in (-1, 0, -1):
+        ls.one_launch(polls)
+        x, st = pcg(b, rel_tol=0.0, max_iter=4)
+        it = [pcg(b, rel_tol=1e-8, use_rz=rz)[1].iterations for rz in (True, False)]
+        runs.append((x, st, it))
+    print(f"[ways] nb={nb} {pc} {prec} it={[r[2] for r in runs]} "
+          f"diff={rel(runs[0][0], runs[1][0]):.2e}", flush=True)
+    assert [r[1].one_launch for r in runs] == [1, 0, 1]
+    assert runs[0][2] == runs[1][2] == runs[2][2]
+    assert np.array_equal(runs[0][0], runs[2][0])
+    # sums in another order: at the precision of the vectors, and with FP32
+    # inverses of the preconditioner's products, amplified by three steps
+    assert rel(runs[0][0], runs[1][0]) < (1e-6 if prec == "fp32" else 1e-13)
+    with pytest.raises(sgipc.SgipcError):
+        ls.one_launch(-2)
