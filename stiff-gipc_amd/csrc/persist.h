@@ -23,11 +23,16 @@ class PersistPlan
     {
         SG_CHECK(n >= -1, -1, "the number of polls is -1, 0 or positive");
         polls = n < 0 ? kPolls : n;
+        pause = skip = 0;
     }
 
-    // some seconds
-    static constexpr int kPolls = 1 << 22;
+    // about a second; the workgroups meet within microseconds once all of them run
+    static constexpr int kPolls = 1 << 20;
     int polls = kPolls;
+    // After a wait that ran out the next solves, 16 and doubling up to 1024 while
+    // it happens again, do not try: each attempt costs kPolls polls, and what kept
+    // a workgroup from running (another program's work on the device) may last.
+    int pause = 0, skip = 0;
 
     int groups = 0;                            // workgroups (0: not this way)
     int rows = 0, halo = 0, banks = 0;         // most of one workgroup
@@ -48,7 +53,7 @@ struct PersistResult
 };
 
 // true: the solve ran (result in *res, x complete); false: this system or
-// device does not take it, nothing was launched
+// device does not take it, or a wait ran out, and x is still to be solved for
 bool persist_solve(PersistPlan& plan, const SysView& S, Mas* mas, const double* dinv,
                    const double* b, double* x, double* z, double* p0, double* p1,
                    const PcgConfig& cfg, int maxit, int every, PersistResult* res, hipStream_t s);

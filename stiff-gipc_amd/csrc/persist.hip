@@ -29,8 +29,9 @@
 // means having the sum; every workgroup adds the partials in the same order.
 // Two sets of words alternate: a workgroup stores into a set again only after
 // a barrier that all have left the set's previous use for.  Waits are bounded:
-// a workgroup that runs out of polls raises ctl[1] = 3 and leaves, and the
-// others follow at their next wait.
+// a workgroup that runs out of polls leaves, the others follow at their next
+// wait, and each sets ctl[2]; the caller then solves with a launch per
+// operation.
 #include "persist.h"
 
 #include <algorithm>
@@ -989,6 +990,11 @@ bool persist_solve(PersistPlan& P, const SysView& S, Mas* mas, const double* din
 {
     if(!P.ready())
         return false;
+    if(P.skip > 0)
+    {
+        P.skip--;
+        return false;
+    }
     const bool contact = S.coo && S.coo->cap > 0 && S.coo->live > 0;
     auto       run     = [&](auto zero, auto is_mas) {
         using T             = decltype(zero);
@@ -1022,7 +1028,13 @@ bool persist_solve(PersistPlan& P, const SysView& S, Mas* mas, const double* din
     SG_HIP(hipMemcpyAsync(hc, P.ctl.data(), sizeof(hc), hipMemcpyDeviceToHost, s));
     SG_HIP(hipMemcpyAsync(ho, P.out.data(), sizeof(ho), hipMemcpyDeviceToHost, s));
     SG_HIP(hipStreamSynchronize(s));
-    SG_CHECK(hc[2] == 0, SGIPC_EHIP, "PCG: a workgroup's wait at the grid barrier ran out");
+    if(hc[2] != 0)  // a wait ran out: every workgroup has left
+    {
+        P.pause = P.pause ? std::min(2 * P.pause, 1024) : 16;
+        P.skip  = P.pause;
+        return false;
+    }
+    P.pause = 0;
     res->stop_at = hc[0];
     res->bad     = hc[1];
     res->rz0     = ho[0];

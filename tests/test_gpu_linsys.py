@@ -393,3 +393,28 @@ def test_pcg_ways_agree(oracle, nb, pc, prec, noalloc):
     assert rel(runs[0][0], runs[1][0]) < (1e-6 if prec == "fp32" else 1e-13)
     with pytest.raises(sgipc.SgipcError):
         ls.one_launch(-2)
+
+
+@pytest.mark.parametrize("noalloc", [False, True])
+@pytest.mark.parametrize("pc", ["mas", "diag"])
+def test_pcg_wait_runs_out(oracle, pc, noalloc):
+    """One poll is too few for over a hundred workgroups to meet: they leave,
+    and the solve is done with a launch per operation, the following ones
+    without trying; a new bound tries again."""
+    import sgipc
+    A, part, b = _spd_system(oracle, 8200, 1)
+    ls = sgipc.LinearSystem(A.rowptr, A.cols, A.vals, part,
+                            sgipc.SGIPC_PRECOND_MAS if pc == "mas" else sgipc.SGIPC_PRECOND_DIAG)
+    pcg = ls.pcg_noalloc if noalloc else ls.pcg
+    ls.one_launch(0)
+    x0, s0 = pcg(b, rel_tol=1e-8)
+    ls.one_launch(1)
+    for _ in range(2):
+        x1, s1 = pcg(b, rel_tol=1e-8)
+        assert s1.converged and s1.one_launch == 0 and s1.iterations == s0.iterations
+        assert np.array_equal(x0, x1)
+    ls.one_launch()
+    x2, s2 = pcg(b, rel_tol=1e-8)
+    assert s2.one_launch == 1 and s2.iterations == s0.iterations
+    # sums in another order, up to where the solves stop
+    assert rel(x2, x0) < 1e-9
