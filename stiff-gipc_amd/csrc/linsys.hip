@@ -1067,12 +1067,12 @@ PcgStats Pcg::solve_t(const SysView& S, Precond pc, Mas* mas, const V* b, V* x,
     PcgVecs<V>& W     = vecs<V>();
     ensure(n);
     W.ensure(n);
+    if(pc == Precond::Diag)
+        build_diag(*S.A, s);
     if constexpr(sizeof(V) == sizeof(double))
         if(!b64 && S.plan && S.plan->ready() && (pc == Precond::Mas || nbody_ == 0))
         {
             // the whole solve in one launch (persist.hip)
-            if(pc == Precond::Diag)
-                build_diag(*S.A, s);
             PersistResult pr;
             if(persist_solve(*S.plan, S, pc == Precond::Mas ? mas : nullptr, dinv_.data(), b, x,
                              W.z.data(), W.p[0].data(), W.p[1].data(), cfg, maxit, every, &pr, s))
@@ -1097,18 +1097,14 @@ PcgStats Pcg::solve_t(const SysView& S, Precond pc, Mas* mas, const V* b, V* x,
     SG_HIP(hipMemsetAsync(ctl_d_.data(), 0, ctl_d_.size() * sizeof(double), s));
     SG_HIP(hipMemsetAsync(x, 0, n * sizeof(V), s));
     SG_HIP(hipMemcpyAsync(W.r.data(), b, n * sizeof(V), hipMemcpyDeviceToDevice, s));
-    if(pc == Precond::Diag)
+    if(pc == Precond::Diag && sizeof(V) == sizeof(float))
     {
-        build_diag(*S.A, s);
-        if(sizeof(V) == sizeof(float))
+        dinv32_.resize(dinv_.size());
+        convert<double, float>((long long)dinv_.size(), dinv_.data(), dinv32_.data(), s);
+        if(nbody_ > 0)
         {
-            dinv32_.resize(dinv_.size());
-            convert<double, float>((long long)dinv_.size(), dinv_.data(), dinv32_.data(), s);
-            if(nbody_ > 0)
-            {
-                binv32_.resize(binv_.size());
-                convert<double, float>((long long)binv_.size(), binv_.data(), binv32_.data(), s);
-            }
+            binv32_.resize(binv_.size());
+            convert<double, float>((long long)binv_.size(), binv_.data(), binv32_.data(), s);
         }
     }
     const int* done = ctl_.data();

@@ -107,9 +107,10 @@ struct PersistArgs
     double rel2, abs2, q_ref;
     int    use_rz, maxit, every;
     u64*    slots;
-    int*    ctl;
-    double* out;
-    int     polls;
+    int*     ctl;
+    double*  out;
+    int      polls;
+    unsigned lds;  // bytes of a workgroup's LDS
 };
 
 struct Barrier
@@ -872,8 +873,9 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
         A.x[3 * (size_t)v0 + i] = xl[i];
 }
 
+// the rest of the arguments; false: the LDS of a compute unit does not hold it
 template <typename T, bool MAS>
-bool launch(PersistPlan& P, Mas* mas, PersistArgs<T> a, hipStream_t s)
+bool fit(const PersistPlan& P, Mas* mas, PersistArgs<T>& a)
 {
     if constexpr(MAS)
     {
@@ -894,17 +896,26 @@ bool launch(PersistPlan& P, Mas* mas, PersistArgs<T> a, hipStream_t s)
         return false;
     a.keep_off     = (int)fix;
     a.cache        = MAS ? (int)((kPLds - fix) / sizeof(T)) : 0;
-    const size_t n = MAS ? kPLds : fix;
-    void*        args[] = {&a};
-    const void*  f      = P.rows <= kPassRows
-                              ? reinterpret_cast<const void*>(&k_pcg_persist<T, MAS, 1>)
-                              : reinterpret_cast<const void*>(&k_pcg_persist<T, MAS, 2>);
-    if(hipLaunchCooperativeKernel(f, dim3(P.groups), dim3(kPT), args, (unsigned)n, s)
-       != hipSuccess)
+    a.lds          = (unsigned)(MAS ? kPLds : fix);
+    return true;
+}
+
+// false: the workgroups do not all fit on the device; any other error is an error
+template <typename T, bool MAS>
+bool launch(PersistPlan& P, PersistArgs<T> a, hipStream_t s)
+{
+    void*       args[] = {&a};
+    const void* f      = P.rows <= kPassRows
+                             ? reinterpret_cast<const void*>(&k_pcg_persist<T, MAS, 1>)
+                             : reinterpret_cast<const void*>(&k_pcg_persist<T, MAS, 2>);
+    const hipError_t e = hipLaunchCooperativeKernel(f, dim3(P.groups), dim3(kPT), args, a.lds, s);
+    if(e == hipErrorCooperativeLaunchTooLarge)
     {
         (void)hipGetLastError();
+        P.groups = 0;  // nor will they for the next solve
         return false;
     }
+    SG_HIP(e);
     return true;
 }
 }  // namespace
@@ -1013,11 +1024,13 @@ bool persist_solve(PersistPlan& P, const SysView& S, Mas* mas, const double* din
         a.rel2 = cfg.rel_tol * cfg.rel_tol, a.abs2 = cfg.abs_tol * cfg.abs_tol;
         a.q_ref = cfg.q_ref, a.use_rz = cfg.use_rz ? 1 : 0, a.maxit = maxit, a.every = every;
         a.slots = P.slots.data(), a.ctl = P.ctl.data(), a.out = P.out.data(), a.polls = P.polls;
-        return launch<T, MAS>(P, mas, a, s);
+        if(!fit<T, MAS>(P, mas, a))
+            return false;
+        SG_HIP(hipMemsetAsync(P.slots.data(), 0, P.slots.size() * sizeof(u64), s));
+        SG_HIP(hipMemsetAsync(P.ctl.data(), 0, P.ctl.size() * sizeof(int), s));
+        SG_HIP(hipMemsetAsync(P.out.data(), 0, P.out.size() * sizeof(double), s));
+        return launch<T, MAS>(P, a, s);
     };
-    SG_HIP(hipMemsetAsync(P.slots.data(), 0, P.slots.size() * sizeof(u64), s));
-    SG_HIP(hipMemsetAsync(P.ctl.data(), 0, P.ctl.size() * sizeof(int), s));
-    SG_HIP(hipMemsetAsync(P.out.data(), 0, P.out.size() * sizeof(double), s));
     const bool ran = !mas          ? run(0.0, std::false_type{})
                      : mas->fp32() ? run(0.0f, std::true_type{})
                                    : run(0.0, std::true_type{});
