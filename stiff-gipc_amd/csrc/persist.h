@@ -1,5 +1,5 @@
-// persist.h -- the FP64 PCG solve of a small or medium system as one
-// cooperative launch (persist.hip).
+// persist.h -- the FP64 PCG solve of a small or medium system as one launch
+// (persist.hip).
 #pragma once
 
 #include "linsys.h"
@@ -35,6 +35,7 @@ class PersistPlan
     int pause = 0, skip = 0;
 
     int groups = 0;                            // workgroups (0: not this way)
+    int dev = 0, units = 0;                    // device, its compute units per XCD
     int rows = 0, halo = 0, banks = 0;         // most of one workgroup
     DBuf<int>            rstart, bstart;       // groups + 1: rows, level-0 banks
     DBuf<int>            hptr, hcol;           // groups + 1; halo columns

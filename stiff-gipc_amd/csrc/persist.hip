@@ -1,4 +1,4 @@
-// persist.hip -- FP64 PCG in one cooperative launch.
+// persist.hip -- FP64 PCG in one launch.
 //
 // The iteration is solve_t's (linsys.hip), the reference's (pcg_solver.cu:
 // 171-304).  With one launch per operation an iteration of a system that does
@@ -35,6 +35,9 @@
 #include "persist.h"
 
 #include <algorithm>
+#include <condition_variable>
+#include <mutex>
+#include <optional>
 
 #include "../../include/sgipc.h"
 #include "mas_tail.h"
@@ -900,36 +903,88 @@ bool fit(const PersistPlan& P, Mas* mas, PersistArgs<T>& a)
     return true;
 }
 
-// false: the workgroups do not all fit on the device; any other error is an error
 template <typename T, bool MAS>
-bool launch(PersistPlan& P, PersistArgs<T> a, hipStream_t s)
+void launch(const PersistPlan& P, PersistArgs<T> a, hipStream_t s)
 {
     void*       args[] = {&a};
     const void* f      = P.rows <= kPassRows
                              ? reinterpret_cast<const void*>(&k_pcg_persist<T, MAS, 1>)
                              : reinterpret_cast<const void*>(&k_pcg_persist<T, MAS, 2>);
-    const hipError_t e = hipLaunchCooperativeKernel(f, dim3(P.groups), dim3(kPT), args, a.lds, s);
-    if(e == hipErrorCooperativeLaunchTooLarge)
-    {
-        (void)hipGetLastError();
-        P.groups = 0;  // nor will they for the next solve
-        return false;
-    }
-    SG_HIP(e);
-    return true;
+    SG_HIP(hipLaunchKernel(f, dim3(P.groups), dim3(kPT), args, a.lds, s));
 }
+
+// The workgroups of a solve wait for each other, so all of them have to run at
+// once.  A workgroup takes a compute unit (its LDS leaves no room for a second
+// one), other kernels end and give theirs back, and the solves of this process
+// share the units out here: a solve holds its units from before its launch
+// until it has ended, and the next one in line waits until enough are free.
+// Workgroups go to the XCDs in turn, so units are counted per XCD; within one,
+// kernels of several streams were seen to fill it to the last unit (101 + 101,
+// 63 + 63 + 63 + 63 and 248 + 6 workgroups on 256 units start within 10 us).  A
+// cooperative launch would have the runtime run one such solve at a time.  ms
+// per solve of several threads with a system each, cooperative launches / this /
+// a launch per operation: 425 rows, 8 threads 0.95-1.05 / 0.37-0.40 / 0.60-0.72;
+// 6,480 rows, 4 threads 1.58 / 1.18 / 1.73, 8 threads (whose streams share
+// hardware queues) 1.59 / 1.2-1.5 / 1.00; 46,656 rows, 8 threads 3.1 / 3.1 / 3.6.
+class Units
+{
+  public:
+    void take(int n, int all)
+    {
+        std::unique_lock<std::mutex> lock(m_);
+        const u64 me = last_++;
+        cv_.wait(lock, [&] { return me == turn_ && used_ + n <= all; });
+        used_ += n;
+        turn_++;
+        cv_.notify_all();
+    }
+    void give(int n)
+    {
+        std::lock_guard<std::mutex> lock(m_);
+        used_ -= n;
+        cv_.notify_all();
+    }
+    static Units& of(int dev)
+    {
+        static Units* const u = new Units[kMaxDevices];  // outlives threads at exit
+        SG_CHECK(dev >= 0 && dev < kMaxDevices, -1, "device index out of range");
+        return u[dev];
+    }
+
+  private:
+    static constexpr int    kMaxDevices = 64;
+    std::mutex              m_;
+    std::condition_variable cv_;
+    int                     used_ = 0;
+    u64                     last_ = 0, turn_ = 0;  // the line's end and head
+};
+
+struct UnitsHeld
+{
+    Units& u;
+    int    n;
+    UnitsHeld(const PersistPlan& P)
+        : u(Units::of(P.dev))
+        , n(std::min((P.groups + kXcds - 1) / kXcds, P.units))
+    {
+        u.take(n, P.units);
+    }
+    ~UnitsHeld() { u.give(n); }
+    UnitsHeld(const UnitsHeld&)            = delete;
+    UnitsHeld& operator=(const UnitsHeld&) = delete;
+};
 }  // namespace
 
 void PersistPlan::build(const Bsr& A, const std::vector<int>& part_first, hipStream_t s)
 {
     groups       = 0;
     const int nb = A.nb;
-    int       dev = 0, cus = 0, coop = 0;
+    int       cus = 0;
     SG_HIP(hipGetDevice(&dev));
     SG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    SG_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
-    const int G = std::min(std::min(kMaxGroups, cus), std::max(1, nb / kGroupRows));
-    if(!coop || nb > kMaxRows * G)
+    units       = cus / kXcds;
+    const int G = std::min(std::min(kMaxGroups, units * kXcds), std::max(1, nb / kGroupRows));
+    if(nb > kMaxRows * G)
         return;
     // row ranges, cut at parts; a bank weighs as much as kBankRows rows
     const bool       mas = !part_first.empty();
@@ -1007,7 +1062,8 @@ bool persist_solve(PersistPlan& P, const SysView& S, Mas* mas, const double* din
         return false;
     }
     const bool contact = S.coo && S.coo->cap > 0 && S.coo->live > 0;
-    auto       run     = [&](auto zero, auto is_mas) {
+    std::optional<UnitsHeld> held;
+    auto run = [&](auto zero, auto is_mas) {
         using T             = decltype(zero);
         constexpr bool MAS  = decltype(is_mas)::value;
         PersistArgs<T> a{};
@@ -1026,10 +1082,12 @@ bool persist_solve(PersistPlan& P, const SysView& S, Mas* mas, const double* din
         a.slots = P.slots.data(), a.ctl = P.ctl.data(), a.out = P.out.data(), a.polls = P.polls;
         if(!fit<T, MAS>(P, mas, a))
             return false;
+        held.emplace(P);
         SG_HIP(hipMemsetAsync(P.slots.data(), 0, P.slots.size() * sizeof(u64), s));
         SG_HIP(hipMemsetAsync(P.ctl.data(), 0, P.ctl.size() * sizeof(int), s));
         SG_HIP(hipMemsetAsync(P.out.data(), 0, P.out.size() * sizeof(double), s));
-        return launch<T, MAS>(P, a, s);
+        launch<T, MAS>(P, a, s);
+        return true;
     };
     const bool ran = !mas          ? run(0.0, std::false_type{})
                      : mas->fp32() ? run(0.0f, std::true_type{})

@@ -418,3 +418,61 @@ def test_pcg_wait_runs_out(oracle, pc, noalloc):
     assert s2.one_launch == 1 and s2.iterations == s0.iterations
     # sums in another order, up to where the solves stop
     assert rel(x2, x0) < 1e-9
+
+
+def test_pcg_threads_one_launch_each(oracle):
+    """Solves of eight threads, together more workgroups than the device holds
+    at once: every one runs as one launch and ends where it does alone."""
+    import threading
+    import sgipc
+    rows = [300, 700, 2100, 4000, 8200, 8200, 17000, 33000]
+    sys_ = []
+    for k, nb in enumerate(rows):
+        A, part, b = _spd_system(oracle, nb, 10 + k)
+        pc = sgipc.SGIPC_PRECOND_DIAG if k == 4 else sgipc.SGIPC_PRECOND_MAS
+        ls = sgipc.LinearSystem(A.rowptr, A.cols, A.vals, part, pc)
+        sys_.append((ls, b, ls.pcg(b, rel_tol=1e-8)))
+    bad = []
+
+    def work(ls, b, alone):
+        try:
+            for _ in range(12):
+                x, st = ls.pcg(b, rel_tol=1e-8)
+                if st.one_launch != 1 or not np.array_equal(x, alone[0]):
+                    bad.append((ls.nb, st.one_launch, rel(x, alone[0])))
+        except Exception as e:  # reported by the main thread
+            bad.append(repr(e))
+    th = [threading.Thread(target=work, args=s) for s in sys_]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not bad, bad[:4]
+
+
+def test_pcg_small_solves_of_threads_overlap(oracle):
+    """Four threads with a small system each (a few workgroups) take less than
+    the solves would one after the other; best of five."""
+    import threading
+    import time
+    import sgipc
+    A, part, b = _spd_system(oracle, 425, 3)
+    own = [sgipc.LinearSystem(A.rowptr, A.cols, A.vals, part) for _ in range(4)]
+
+    def run(ls):
+        for _ in range(20):
+            assert ls.pcg(b, rel_tol=0.0, max_iter=201)[1].one_launch == 1
+
+    def timed(systems):
+        th = [threading.Thread(target=run, args=(ls,)) for ls in systems]
+        t0 = time.perf_counter()
+        for t in th:
+            t.start()
+        for t in th:
+            t.join()
+        return time.perf_counter() - t0
+    for ls in own:
+        run(ls)
+    ratio = min(timed(own) / timed(own[:1]) for _ in range(5))
+    print(f"[threads] four threads / one = {ratio:.2f}", flush=True)
+    assert ratio < 2.5
