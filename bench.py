@@ -292,7 +292,7 @@ def main():
             f"steps_begun={adv['time_steps_begun']} capped={adv['capped_steps']} "
             f"fallbacks={adv['solver_fallbacks']}")
         kern[name] = {}
-        for kname in ("spmv", "mas_apply_l0", "fem", "mas_invert"):
+        for kname in ("spmv", "mas_apply_l0", "fem", "mas_invert", "pcg"):
             nl, tot = sim.profile_query(kname)
             if nl:
                 kern[name][kname] = (nl, tot)
@@ -309,12 +309,19 @@ def main():
     # ---- roofline of the dominant profiled kernel of the value mode
     fp32 = value_mode.startswith("mixed")
     hbm = {k: v for k, v in kern[value_mode].items() if k in ("spmv", "mas_apply_l0")}
+    # FP64 solves as one launch have neither of the two: priced as one kernel,
+    # both parts' bytes for each of its iterations (the mean of the timed solves)
+    if not hbm and "pcg" in kern[value_mode]:
+        hbm = {"pcg": kern[value_mode]["pcg"]}
     roof = None
     if hbm:
         dom = max(hbm, key=lambda k: hbm[k][1])
         nl, tot = hbm[dom]
         avg_s = tot / nl * 1e-3
         byt = algorithmic_bytes(dom, sz, nparts, fp32)
+        if dom == "pcg":
+            byt = adv["pcg_iterations"] / args.steps * sum(
+                algorithmic_bytes(k, sz, nparts, False) for k in ("spmv", "mas_apply_l0"))
         ach = byt / avg_s / 1e9
         default_shape = (args.settle == settle_default and args.n_side == 4 and args.cells == 8
                          and not args.morton)

@@ -345,7 +345,9 @@ typedef struct sgipc_advance_stats {
 int sgipc_advance(sgipc_t ctx, int32_t n, sgipc_advance_stats* stats);
 
 /* Per-kernel device timing with HIP events on the library stream.
- * Names: "spmv" (PCG A p), "mas_apply_l0", "fem", "mas_invert".
+ * Names: "spmv" (PCG A p), "mas_apply_l0", "fem", "mas_invert", "pcg" (an FP64
+ * solve as one launch; such a solve has no launches of the first two, which
+ * sgipc_one_launch(ctx, 0) brings back).
  * every >= 1 clears and starts collection, timing every every-th launch of
  * each name (an event pair costs microseconds of stream time); 0 stops it.
  * query returns the number of timed launches and their summed duration. */

@@ -1075,7 +1075,8 @@ PcgStats Pcg::solve_t(const SysView& S, Precond pc, Mas* mas, const V* b, V* x,
             // the whole solve in one launch (persist.hip)
             PersistResult pr;
             if(persist_solve(*S.plan, S, pc == Precond::Mas ? mas : nullptr, dinv_.data(), b, x,
-                             W.z.data(), W.p[0].data(), W.p[1].data(), cfg, maxit, every, &pr, s))
+                             W.z.data(), W.p[0].data(), W.p[1].data(), cfg, maxit, every, &pr, s,
+                             prof))
             {
                 PcgStats st;
                 st.one_launch = true;

@@ -57,6 +57,7 @@ struct PersistResult
 // device does not take it, or a wait ran out, and x is still to be solved for
 bool persist_solve(PersistPlan& plan, const SysView& S, Mas* mas, const double* dinv,
                    const double* b, double* x, double* z, double* p0, double* p1,
-                   const PcgConfig& cfg, int maxit, int every, PersistResult* res, hipStream_t s);
+                   const PcgConfig& cfg, int maxit, int every, PersistResult* res, hipStream_t s,
+                   Profiler* prof);
 
 }  // namespace sgipc

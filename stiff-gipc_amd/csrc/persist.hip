@@ -904,13 +904,15 @@ bool fit(const PersistPlan& P, Mas* mas, PersistArgs<T>& a)
 }
 
 template <typename T, bool MAS>
-void launch(const PersistPlan& P, PersistArgs<T> a, hipStream_t s)
+void launch(const PersistPlan& P, PersistArgs<T> a, std::pair<hipEvent_t, hipEvent_t> ev,
+            hipStream_t s)
 {
     void*       args[] = {&a};
     const void* f      = P.rows <= kPassRows
                              ? reinterpret_cast<const void*>(&k_pcg_persist<T, MAS, 1>)
                              : reinterpret_cast<const void*>(&k_pcg_persist<T, MAS, 2>);
-    SG_HIP(hipLaunchKernel(f, dim3(P.groups), dim3(kPT), args, a.lds, s));
+    SG_HIP(hipExtLaunchKernel(f, dim3(P.groups), dim3(kPT), args, a.lds, s, ev.first, ev.second,
+                              0));
 }
 
 // The workgroups of a solve wait for each other, so all of them have to run at
@@ -1052,7 +1054,8 @@ void PersistPlan::build(const Bsr& A, const std::vector<int>& part_first, hipStr
 
 bool persist_solve(PersistPlan& P, const SysView& S, Mas* mas, const double* dinv,
                    const double* b, double* x, double* z, double* p0, double* p1,
-                   const PcgConfig& cfg, int maxit, int every, PersistResult* res, hipStream_t s)
+                   const PcgConfig& cfg, int maxit, int every, PersistResult* res, hipStream_t s,
+                   Profiler* prof)
 {
     if(!P.ready())
         return false;
@@ -1086,7 +1089,10 @@ bool persist_solve(PersistPlan& P, const SysView& S, Mas* mas, const double* din
         SG_HIP(hipMemsetAsync(P.slots.data(), 0, P.slots.size() * sizeof(u64), s));
         SG_HIP(hipMemsetAsync(P.ctl.data(), 0, P.ctl.size() * sizeof(int), s));
         SG_HIP(hipMemsetAsync(P.out.data(), 0, P.out.size() * sizeof(double), s));
-        launch<T, MAS>(P, a, s);
+        launch<T, MAS>(P, a,
+                       prof ? prof->kernel_events("pcg")
+                            : std::pair<hipEvent_t, hipEvent_t>{nullptr, nullptr},
+                       s);
         return true;
     };
     const bool ran = !mas          ? run(0.0, std::false_type{})

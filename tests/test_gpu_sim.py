@@ -262,3 +262,38 @@ def test_newton_mixed_precision_tracks_fp64(oracle):
         out[prec] = xs
     for a, b in zip(out[sgipc.SGIPC_SOLVE_FP64], out[sgipc.SGIPC_SOLVE_MIXED]):
         assert np.abs(a - b).max() / np.abs(a).max() < 1e-6
+
+
+def test_profile_of_a_solve_as_one_launch():
+    """A FP64 solve as one launch is one launch of "pcg"; as a launch per
+    operation, and in the mixed mode, "spmv" and "mas_apply_l0" are timed.  The
+    Newton iterate from one state is the same both ways up to rounding."""
+    import sgipc
+    from sgipc import scene as S
+    sc = S.bar_scene()
+    sim = sgipc.Simulation(sc)
+    sim.set_positions(sc.x + 0.003 * np.random.default_rng(0).normal(size=sc.x.shape))
+    state = (sim.positions(), sim.velocities(), sim.xtilde(), sim.kappa)
+    names = ("pcg", "spmv", "mas_apply_l0", "mas_invert")
+
+    def run(polls, precision):
+        sim.one_launch(polls)
+        sim.set_pcg(rel_tol=1e-6, use_rz=False, solver_precision=precision)
+        sim.set_state(*state)
+        sim.profile(1)
+        it = sim.newton_iteration()["pcg_iterations"]
+        q = {k: sim.profile_query(k) for k in names}
+        sim.profile(0)
+        print(f"[profile] polls={polls} mixed={precision} it={it} {q}", flush=True)
+        assert all((n > 0) == (ms > 0.0) for n, ms in q.values())
+        assert q["mas_invert"][0] == 1
+        return it, {k: n for k, (n, _) in q.items()}, sim.positions()
+
+    it, q, x1 = run(-1, sgipc.SGIPC_SOLVE_FP64)
+    assert q["pcg"] == 1 and q["spmv"] == q["mas_apply_l0"] == 0
+    it0, q, x0 = run(0, sgipc.SGIPC_SOLVE_FP64)
+    assert q["pcg"] == 0 and q["spmv"] >= it and q["mas_apply_l0"] >= it and it0 == it
+    # FP32 inverses: the iterates of two orders of sums meet at the stop tolerance
+    assert np.abs(x1 - x0).max() < 1e-6 * np.abs(x1 - state[0]).max()
+    it, q, _ = run(-1, sgipc.SGIPC_SOLVE_MIXED)
+    assert q["pcg"] == 0 and q["spmv"] >= it and q["mas_apply_l0"] >= it
