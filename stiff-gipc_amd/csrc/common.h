@@ -206,6 +206,16 @@ class Profiler
         ent.pending.push_back(p);
         return p;
     }
+    // the launch that the last kernel_events(name) was for does not count
+    void discard(const char* name, std::pair<hipEvent_t, hipEvent_t> p)
+    {
+        if(!p.first)
+            return;
+        auto& ent = e_[name];
+        ent.pending.pop_back();
+        ent.calls--;
+        pool_.push_back(p);
+    }
     void end(const char* name, hipStream_t s)
     {
         if(!enabled)

@@ -54,7 +54,8 @@ struct PersistResult
 };
 
 // true: the solve ran (result in *res, x complete); false: this system or
-// device does not take it, or a wait ran out, and x is still to be solved for
+// device does not take it, its contact rows are better served by a launch per
+// operation, or a wait ran out, and x is still to be solved for
 bool persist_solve(PersistPlan& plan, const SysView& S, Mas* mas, const double* dinv,
                    const double* b, double* x, double* z, double* p0, double* p1,
                    const PcgConfig& cfg, int maxit, int every, PersistResult* res, hipStream_t s,

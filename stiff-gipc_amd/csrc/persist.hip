@@ -65,6 +65,16 @@ constexpr int kGroupRows = 64;
 // alone the workgroups of a 46,656-row system get up to 25 banks, 17 on
 // average, and wait for the largest; with 8 rows per bank up to 22
 constexpr int kBankRows  = 8;
+// Contact blocks of a workgroup's rows beyond the first kPT follow in rounds of
+// kPT, one after the other, while all other workgroups wait; the four lanes of a
+// row sum its part of a round.  A launch per operation instead leaves the
+// longest row to four lanes.  ns: of a round, of a round per block of the
+// longest row in it, of a launch per operation per block of the longest row,
+// and what one launch gains without contact.  us per iteration, one launch / a
+// launch per operation, by blocks of a workgroup and of its longest row: 743,
+// 162: 18 / 28; 1,317, 88: 20 / 26; 1,831, 444: 34 / 42; 2,803, 690: 56 / 55;
+// 4,190, 279: 69 / 38; 4,904, 1,220: 98 / 82; 20,928, 5,184: 461 / 278.
+constexpr int kRoundNs = 4500, kRoundRowNs = 13, kRowNs = 50, kGainNs = 10000;
 constexpr int kSlotWords = 4;              // two doubles in four words
 // R of a 16-node bank in LDS takes 50 entries instead of 48: the members of
 // consecutive clusters lie in consecutive banks, and 48 would put their reads
@@ -298,6 +308,32 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
     Barrier   bar{A.slots, A.groups, b, A.polls, 0u, bar_part, bar_tot, &fail};
     if(tid == 0)
         fail = 0;
+    if(A.rp2)
+    {
+        // a launch per operation is the faster way for some workgroup's contact
+        // rows: all leave
+        int len = tid < nloc ? A.rp2[v0 + tid + 1] - A.rp2[v0 + tid] : 0;
+        for(int o = 32; o > 0; o >>= 1)
+            len = max(len, __shfl_xor(len, o, 64));
+        if(lane == 0)
+            wcnt[w] = len;
+        __syncthreads();
+        for(int q = 0; q < kPW; q++)
+            len = max(len, wcnt[q]);
+        const long long more = (A.rp2[v0 + nloc] - A.rp2[v0] + kPT - 1) / kPT - 1;
+        const bool      over = more > 0
+                          && more * (kRoundNs + kRoundRowNs * min(len, kPT))
+                                 > kGainNs + (long long)kRowNs * len;
+        bar.arrive<1>(tid == 0 && over ? 1.0 : 0.0);
+        double     any = 0.0;
+        const bool met = bar.wait<1>(&any);
+        if(!met || any != 0.0)
+        {
+            if(tid == 0 && (!met || b == 0))
+                A.ctl[met ? 3 : 2] = 1;
+            return;
+        }
+    }
 
     // ---- LDS: [own | halo] p and x, own r, z, A p, then the MAS tail
     const int NL3 = 3 * A.nloc, NV = 3 * (A.nloc + A.nhalo);
@@ -1065,7 +1101,8 @@ bool persist_solve(PersistPlan& P, const SysView& S, Mas* mas, const double* din
         return false;
     }
     const bool contact = S.coo && S.coo->cap > 0 && S.coo->live > 0;
-    std::optional<UnitsHeld> held;
+    std::optional<UnitsHeld>          held;
+    std::pair<hipEvent_t, hipEvent_t> ev{nullptr, nullptr};
     auto run = [&](auto zero, auto is_mas) {
         using T             = decltype(zero);
         constexpr bool MAS  = decltype(is_mas)::value;
@@ -1089,10 +1126,9 @@ bool persist_solve(PersistPlan& P, const SysView& S, Mas* mas, const double* din
         SG_HIP(hipMemsetAsync(P.slots.data(), 0, P.slots.size() * sizeof(u64), s));
         SG_HIP(hipMemsetAsync(P.ctl.data(), 0, P.ctl.size() * sizeof(int), s));
         SG_HIP(hipMemsetAsync(P.out.data(), 0, P.out.size() * sizeof(double), s));
-        launch<T, MAS>(P, a,
-                       prof ? prof->kernel_events("pcg")
-                            : std::pair<hipEvent_t, hipEvent_t>{nullptr, nullptr},
-                       s);
+        if(prof)
+            ev = prof->kernel_events("pcg");
+        launch<T, MAS>(P, a, ev, s);
         return true;
     };
     const bool ran = !mas          ? run(0.0, std::false_type{})
@@ -1109,9 +1145,16 @@ bool persist_solve(PersistPlan& P, const SysView& S, Mas* mas, const double* din
     {
         P.pause = P.pause ? std::min(2 * P.pause, 1024) : 16;
         P.skip  = P.pause;
+    }
+    else
+        P.pause = 0;
+    // or too many contact blocks in one workgroup's rows
+    if(hc[2] != 0 || hc[3] != 0)
+    {
+        if(prof)
+            prof->discard("pcg", ev);
         return false;
     }
-    P.pause = 0;
     res->stop_at = hc[0];
     res->bad     = hc[1];
     res->rz0     = ho[0];

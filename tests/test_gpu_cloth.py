@@ -229,14 +229,16 @@ def test_cloth_over_affine_boxes_mixed_tracks_fp64(oracle):
             assert np.abs(d - d0).max() < 1e-6
 
 
-def test_newton_iteration_with_long_contact_rows(oracle):
+@pytest.mark.parametrize("n,one", [(20, 1), (40, 0)])
+def test_newton_iteration_with_long_contact_rows(oracle, n, one):
     """A sheet lying flat on the top face of a fixed box: the box's few
     vertices carry the contact blocks of the whole sheet, more than a
-    workgroup of the one-launch solve takes in one round.  One Newton
+    workgroup of the one-launch solve takes in one round; with too many
+    rounds a launch per operation is faster and taken.  One Newton
     iteration against the oracle (the scale of the iterates above)."""
     import sgipc
     from sgipc import scene as S
-    sc = S.cloth_scene(n=40, size=0.095, height=0.1013, n_boxes=1)
+    sc = S.cloth_scene(n=n, size=0.095, height=0.1013, n_boxes=1)
     sc.mas_precision = sgipc.SGIPC_MAS_FP64
     sim = sgipc.Simulation(sc)
     w = oracle.World(sc)
@@ -245,11 +247,13 @@ def test_newton_iteration_with_long_contact_rows(oracle):
     _, rowptr, cols, _ = sim.assemble()
     box = np.setdiff1d(np.arange(sc.n_verts), sc.tris)
     far = sum(int(np.isin(cols[rowptr[v]:rowptr[v + 1]], box, invert=True).sum()) for v in box)
+    sim.profile(1)
     st = sim.newton_iteration()
+    launches = {k: sim.profile_query(k)[0] for k in ("pcg", "spmv")}
     so = w.newton_iteration()
     err = np.abs(sim.positions() - w.positions()).max() / np.abs(w.positions()).max()
-    print(f"[cloth-rows] box contact blocks={far} coo={sim.sizes()['coo_blocks']} "
+    print(f"[cloth-rows] n={n} {launches} box contact blocks={far} coo={sim.sizes()['coo_blocks']} "
           f"pcg={st['pcg_iterations']}/{so['pcg_iterations']} err={err:.2e}", flush=True)
-    assert far > 512
+    assert far > 512 and launches["pcg"] == one and (launches["spmv"] == 0) == (one == 1)
     assert abs(st["pcg_iterations"] - so["pcg_iterations"]) <= 10
     assert err < 1e-6
