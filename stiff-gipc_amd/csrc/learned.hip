@@ -435,7 +435,11 @@ __global__ void __launch_bounds__(kHid) k_mlp_backward(int n, MlpW w, const floa
 // launch of its own).
 constexpr int kWgT = 16;   // tile edge
 constexpr int kWgS = 64;   // samples staged at a time
-constexpr int kWg1 = 16, kWg2 = 72, kWg3 = 9, kWgBlocks = kWg1 + kWg2 + kWg3 + 1;
+constexpr int wg_tiles(int n) { return (n + kWgT - 1) / kWgT; }
+constexpr int kWg1 = wg_tiles(kIn + 1) * wg_tiles(kHid);
+constexpr int kWg2 = wg_tiles(kHid + 1) * wg_tiles(kHid);
+constexpr int kWg3 = wg_tiles(kHid + 1) * wg_tiles(kOut);
+constexpr int kWgBlocks = kWg1 + kWg2 + kWg3 + 1;
 
 __global__ void __launch_bounds__(256) k_mlp_wgrad(int n, const float* __restrict__ X,
                                                    const float* __restrict__ H1,
@@ -470,7 +474,7 @@ __global__ void __launch_bounds__(256) k_mlp_wgrad(int n, const float* __restric
         A = H1, lda = kHid, G = dH2, ldg = kHid, ow = kOffW2, ob = kOffB2;
     else
         b -= kWg2, A = H2, lda = kHid, G = dY, ldg = kOut, ow = kOffW3, ob = kOffB3;
-    const int tj = (ldg + kWgT - 1) / kWgT;  // tiles along the outputs
+    const int tj = wg_tiles(ldg);  // tiles along the outputs
     const int i0 = kWgT * (b / tj), j0 = kWgT * (b % tj);
     const int ti = t / kWgT, tx = t % kWgT;
     __shared__ float As[kWgS][kWgT + 1], Gs[kWgS][kWgT + 1];

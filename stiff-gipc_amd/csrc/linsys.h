@@ -165,7 +165,7 @@ class MasGalerkin
 template <typename T>
 struct MasView
 {
-    const int *     vert_of_slot, *going_next, *bank_first, *bank_ncl, *chain, *child_bank;
+    const int *     vert_of_slot, *bank_first, *bank_ncl, *chain, *child_bank;
     const unsigned* child_mask;
     const T *       inv, *dense;  // packed; coarse banks dense
     T *             R, *Z;

@@ -17,9 +17,9 @@
 //     _schwarzLocalXSym6 :954, __collectFinalZ_new :848).
 //
 // MI355X design: a 16-node bank is a quarter of a wave64; closures run on a
-// bank's 16 lanes through LDS, counts come from one 64-bit ballot.  Coarse
-// Galerkin sums use wave-aggregated atomics (one atomic per distinct target
-// per wave).  Each bank matrix is inverted by one wave in LDS (lane = column).
+// bank's 16 lanes through LDS, counts come from one 64-bit ballot.  The coarse
+// bank matrices are summed in sorted order (mas_galerkin.hip), every bank matrix
+// is inverted by one wave (mas_invert.hip; here the tiled FP64-MFMA variant).
 // The apply is level-synchronous and atomic-free: every node of level l+1 lies
 // inside a single bank of level l, so restriction is a bank-local LDS
 // reduction done by the same wave that applies that bank's inverse.
@@ -1180,16 +1180,16 @@ void Mas::apply(const double* r, double* z, hipStream_t s)
 template <>
 MasView<float> Mas::view<float>()
 {
-    return {vert_of_slot_.data(), going_next_.data(), bank_first_.data(), bank_ncl_.data(),
-            chain_.data(), child_bank_.data(), child_mask_.data(), inv32_.data(), dense32_.data(), R32_.data(),
-            Z32_.data()};
+    return {vert_of_slot_.data(), bank_first_.data(), bank_ncl_.data(), chain_.data(),
+            child_bank_.data(),   child_mask_.data(), inv32_.data(),    dense32_.data(),
+            R32_.data(),          Z32_.data()};
 }
 template <>
 MasView<double> Mas::view<double>()
 {
-    return {vert_of_slot_.data(), going_next_.data(), bank_first_.data(), bank_ncl_.data(),
-            chain_.data(), child_bank_.data(), child_mask_.data(), inv64_.data(), dense64_.data(), R64_.data(),
-            Z64_.data()};
+    return {vert_of_slot_.data(), bank_first_.data(), bank_ncl_.data(), chain_.data(),
+            child_bank_.data(),   child_mask_.data(), inv64_.data(),    dense64_.data(),
+            R64_.data(),          Z64_.data()};
 }
 
 std::vector<int> Mas::chain_host(hipStream_t s) const
