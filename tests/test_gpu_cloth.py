@@ -257,3 +257,35 @@ def test_newton_iteration_with_long_contact_rows(oracle, n, one):
     assert far > 512 and launches["pcg"] == one and (launches["spmv"] == 0) == (one == 1)
     assert abs(st["pcg_iterations"] - so["pcg_iterations"]) <= 10
     assert err < 1e-6
+
+
+@pytest.mark.parametrize("name", ["sheet", "stack", "affine"])
+def test_contact_solve_ways_agree(name):
+    """From one state in contact, a Newton iteration whose solve runs as one
+    launch and as a launch per operation: three PCG iterations with FP64
+    inverses end at the same positions up to rounding (contact blocks are summed
+    by atomics, in an order that varies too)."""
+    import sgipc
+    from sgipc import scene as S
+    sc = {"sheet": lambda: S.cloth_scene(n=20, size=0.095, height=0.1013, n_boxes=1),
+          "stack": lambda: S.stack_scene(n=3, cells=4, friction_mu=0.2),
+          "affine": lambda: S.abd_scene(n_abd=3, cells=3)}[name]()
+    sc.mas_precision = sgipc.SGIPC_MAS_FP64
+    sim = sgipc.Simulation(sc)
+    sim.kappa = 1e4
+    sim.set_pcg(rel_tol=0.0, max_iter=4)
+    state = (sim.positions(), sim.velocities(), sim.xtilde(), sim.kappa)
+    x = {}
+    for polls in (-1, 0):
+        sim.one_launch(polls)
+        sim.set_state(*state)
+        sim.profile(1)
+        st = sim.newton_iteration()
+        assert sim.profile_query("pcg")[0] == (1 if polls else 0)
+        x[polls] = sim.positions() - state[0]
+    err = np.abs(x[-1] - x[0]).max() / np.abs(x[0]).max()
+    print(f"[ways-contact] {name} coo={sim.sizes()['coo_blocks']} pairs={st['n_pairs']} "
+          f"ground={st['n_ground']} step={np.abs(x[0]).max():.2e} diff={err:.2e}", flush=True)
+    assert st["n_pairs"] > 0 and np.abs(x[0]).max() > 0.0
+    # positions of about 0.1 round at 1e-17, steps are larger than 1e-6
+    assert err < 1e-10
