@@ -129,10 +129,10 @@ struct PersistArgs
 struct Barrier
 {
     u64*     slots;
-    int      groups, b, polls;
+    int      groups, b;
     unsigned epoch = 0;
     double * part, *tot;  // LDS: 2 kPW each
-    int*     fail;        // LDS
+    int*     fail;        // LDS: a wait ran out, most polls of one
 
     __device__ __forceinline__ u64* words(int g) const
     {
@@ -191,7 +191,7 @@ struct Barrier
 #pragma unroll
                 for(int i = 0; i < M; i++)
                     there = there && (unsigned)q[i] == epoch;
-            } while(!there && ++n < polls);
+            } while(!there && ++n < fail[1]);
             if(!there)
                 *fail = 1;
             if(N > 0)
@@ -294,46 +294,42 @@ size_t persist_lds(int nloc, int nhalo, int nbank, const TailPlan& tp, int L, bo
     return (n + 79) / 16 * 16;
 }
 
+// ctl[3] = 1 if a launch per operation is the faster way for the contact rows of
+// some workgroup of the solve (one wave each).  A launch of its own, 3 us once
+// per solve: inside k_pcg_persist it cost registers in every iteration (46,656
+// rows: 0.7%).
+__global__ void __launch_bounds__(64) k_contact_rows(const int* __restrict__ rstart,
+                                                     const int* __restrict__ rp,
+                                                     int* __restrict__ ctl)
+{
+    const int v0 = rstart[blockIdx.x], v1 = rstart[blockIdx.x + 1];
+    int       len = 0;
+    for(int v = v0 + (int)threadIdx.x; v < v1; v += 64)
+        len = max(len, rp[v + 1] - rp[v]);
+    for(int o = 32; o > 0; o >>= 1)
+        len = max(len, __shfl_xor(len, o, 64));
+    const long long more = (rp[v1] - rp[v0] + kPT - 1) / kPT - 1;
+    if(threadIdx.x == 0 && more > 0
+       && more * (kRoundNs + kRoundRowNs * min(len, kPT)) > kGainNs + (long long)kRowNs * len)
+        ctl[3] = 1;
+}
+
 template <typename T, bool MAS, int kPasses>
 __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
 {
     extern __shared__ __align__(16) unsigned char plds[];
     __shared__ double bar_part[2 * kPW], bar_tot[2 * kPW];
-    __shared__ int    fail, wcnt[kPW];
+    __shared__ int    fail[2], wcnt[kPW];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int b  = blockIdx.x;
     const int v0 = A.rstart[b], nloc = A.rstart[b + 1] - v0;
     const int h0 = A.hptr[b], nh = A.hptr[b + 1] - h0;
     const int n3 = 3 * nloc;
-    Barrier   bar{A.slots, A.groups, b, A.polls, 0u, bar_part, bar_tot, &fail};
+    Barrier   bar{A.slots, A.groups, b, 0u, bar_part, bar_tot, fail};
     if(tid == 0)
-        fail = 0;
-    if(A.rp2)
-    {
-        // a launch per operation is the faster way for some workgroup's contact
-        // rows: all leave
-        int len = tid < nloc ? A.rp2[v0 + tid + 1] - A.rp2[v0 + tid] : 0;
-        for(int o = 32; o > 0; o >>= 1)
-            len = max(len, __shfl_xor(len, o, 64));
-        if(lane == 0)
-            wcnt[w] = len;
-        __syncthreads();
-        for(int q = 0; q < kPW; q++)
-            len = max(len, wcnt[q]);
-        const long long more = (A.rp2[v0 + nloc] - A.rp2[v0] + kPT - 1) / kPT - 1;
-        const bool      over = more > 0
-                          && more * (kRoundNs + kRoundRowNs * min(len, kPT))
-                                 > kGainNs + (long long)kRowNs * len;
-        bar.arrive<1>(tid == 0 && over ? 1.0 : 0.0);
-        double     any = 0.0;
-        const bool met = bar.wait<1>(&any);
-        if(!met || any != 0.0)
-        {
-            if(tid == 0 && (!met || b == 0))
-                A.ctl[met ? 3 : 2] = 1;
-            return;
-        }
-    }
+        fail[0] = 0, fail[1] = A.polls;
+    if(A.rp2 && A.ctl[3])  // k_contact_rows
+        return;
 
     // ---- LDS: [own | halo] p and x, own r, z, A p, then the MAS tail
     const int NL3 = 3 * A.nloc, NV = 3 * (A.nloc + A.nhalo);
@@ -906,7 +902,7 @@ __global__ void __launch_bounds__(kPT) k_pcg_persist(PersistArgs<T> A)
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load into LDS is under way
     __syncthreads();
-    if(fail && tid == 0)
+    if(fail[0] && tid == 0)
         A.ctl[2] = 1;  // a wait ran out
     for(int i = tid; i < n3; i += kPT)
         A.x[3 * (size_t)v0 + i] = xl[i];
@@ -1126,6 +1122,12 @@ bool persist_solve(PersistPlan& P, const SysView& S, Mas* mas, const double* din
         SG_HIP(hipMemsetAsync(P.slots.data(), 0, P.slots.size() * sizeof(u64), s));
         SG_HIP(hipMemsetAsync(P.ctl.data(), 0, P.ctl.size() * sizeof(int), s));
         SG_HIP(hipMemsetAsync(P.out.data(), 0, P.out.size() * sizeof(double), s));
+        if(contact)
+        {
+            hipLaunchKernelGGL(k_contact_rows, dim3(P.groups), dim3(64), 0, s, a.rstart, a.rp2,
+                               a.ctl);
+            SG_LAUNCH_CHECK();
+        }
         if(prof)
             ev = prof->kernel_events("pcg");
         launch<T, MAS>(P, a, ev, s);
