@@ -6,8 +6,9 @@
 // round trips behind a launch boundary.  Here every workgroup keeps its rows'
 // x, r, z, A p and p in LDS and most of its matrix blocks in registers for the
 // whole solve and meets the others at three grid barriers per iteration: after
-// p.Ap, after the level-1 restriction, after r.z (two with block Jacobi).  A
-// barrier with its exchange is 1.9 us with 2 workgroups, 2.9 us with 32, 4.2 us
+// p.Ap, after the level-1 restriction, after r.z (two with block Jacobi), one
+// more for every coarse level below the tail and one at a check iteration (x for
+// the residual).  A barrier with its exchange is 1.9 us with 2 workgroups, 2.9 us with 32, 4.2 us
 // with 256; they bound the small systems.  The level-0 products run between
 // arriving at the second one and waiting for it; LDS left over keeps the
 // inverse rows of the tail products and level-0 inverses.  Per iteration, a
@@ -295,7 +296,7 @@ size_t persist_lds(int nloc, int nhalo, int nbank, const TailPlan& tp, int L, bo
 }
 
 // ctl[3] = 1 if a launch per operation is the faster way for the contact rows of
-// some workgroup of the solve (one wave each).  A launch of its own, 3 us once
+// some workgroup of the solve (one wave each).  A launch of its own, 5 us once
 // per solve: inside k_pcg_persist it cost registers in every iteration (46,656
 // rows: 0.7%).
 __global__ void __launch_bounds__(64) k_contact_rows(const int* __restrict__ rstart,
